@@ -76,6 +76,12 @@ _SIGNATURES = [
     ("aimg_decode_gemm_bf16", ctypes.c_int,
      [ctypes.POINTER(AimgTensor), ctypes.c_int64, ctypes.c_int64, ctypes.c_void_p, ctypes.c_int,
       ctypes.c_void_p, ctypes.c_void_p]),
+    ("aimg_gemm_workspace_nbytes", ctypes.c_int,
+     [ctypes.POINTER(AimgTensor), ctypes.c_int64, ctypes.c_int64, ctypes.c_int,
+      ctypes.POINTER(ctypes.c_size_t)]),
+    ("aimg_decode_gemm_bf16_ws", ctypes.c_int,
+     [ctypes.POINTER(AimgTensor), ctypes.c_int64, ctypes.c_int64, ctypes.c_void_p, ctypes.c_int,
+      ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
     ("aimg_recombine_bf16", ctypes.c_int,
      [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p]),
     ("aimg_cpu_decode_bf16", ctypes.c_int, [ctypes.POINTER(AimgTensor), ctypes.c_int, ctypes.c_int]),

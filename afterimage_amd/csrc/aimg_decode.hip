@@ -143,8 +143,15 @@ enum Mode : int {
     kModeIndex = 4, // the segment index: each segment's first boundary and codewords
     kModeGemm = 5,      // Y += X W^T for up to 16 rows of X, W decoded on the fly (MFMA)
     kModeGemmRows = 6,  // kModeGemm for rows of more than kGemmPieceMaxCols columns
+    kModeGemmTile = 7,  // kModeGemm through a ring of exponents in a workspace, 16 whole rows at a time
 };
-constexpr bool is_gemm(int mode) { return mode == kModeGemm || mode == kModeGemmRows; }
+constexpr bool is_gemm(int mode) {
+    return mode == kModeGemm || mode == kModeGemmRows || mode == kModeGemmTile;
+}
+// GEMM modes that keep partial sums of a matrix tile from round to round.
+constexpr bool keeps_tile_sums(int mode) { return mode == kModeGemm || mode == kModeGemmRows; }
+// Modes that read sign/mantissa bytes outside the round's own requests.
+constexpr bool reads_sm_late(int mode) { return mode == kModeGemmRows || mode == kModeGemmTile; }
 // Modes that combine the exponents with sign/mantissa bytes.
 constexpr bool needs_sm(int mode) { return mode != kModeU8 && mode != kModeIndex; }
 // Job::ib of a chunk decoded without the index.
@@ -165,6 +172,10 @@ struct GemvArgs {
     int32_t batch;
     uint32_t step_rows;  // 4096 elements (8 per thread of a 512-thread chunk)
     uint32_t step_cols;  // = step_rows rows + step_cols columns
+    // kModeGemmTile: workgroup b's ring is the ring_rows * cols bytes from
+    // ring + b * ring_rows * cols (below 2^31 a workgroup).
+    uint8_t* ring;
+    uint32_t ring_rows;
 };
 
 struct LaunchArgs {
@@ -955,7 +966,7 @@ __device__ __forceinline__ void store_one(const DevTensor& T, const GemvArgs& G,
 // (groups k * tpc + i of the round), requested ahead of use.
 template <int kMode>
 struct SmBatch {
-    uint2 v[needs_sm(kMode) && kMode != kModeGemmRows ? kSmAhead : 1];
+    uint2 v[needs_sm(kMode) && !reads_sm_late(kMode) ? kSmAhead : 1];
 };
 
 // Buffer loads (zero past the tensor's last byte), so the batch needs no
@@ -965,8 +976,8 @@ template <int kMode, int kGroup>
 // without reading memory).
 __device__ __forceinline__ void sm_issue(SmBatch<kMode>& B, const DevTensor& T, int64_t a0,
                                          uint32_t i, uint32_t tpc, uint32_t limit = 0xFFFFFFFFu) {
-    // (kModeGemmRows reads them where its matrix tiles want them.)
-    if (!needs_sm(kMode) || kMode == kModeGemmRows || kGroup == 1) return;
+    // (Some GEMM modes read them where their matrix tiles want them.)
+    if (!needs_sm(kMode) || reads_sm_late(kMode) || kGroup == 1) return;
     const uint32_t n = static_cast<uint32_t>(T.n_symbols);
     const __amdgpu_buffer_rsrc_t rs = buffer_of(T.sm, n < limit ? n : limit);
     const uint32_t v0 = static_cast<uint32_t>(a0) + i * kGroup;
@@ -1470,6 +1481,292 @@ __device__ __forceinline__ void gemm_round_rows(const DevTensor& T, const GemvAr
         reinterpret_cast<uint2*>(stage + nfull * 8)[1] = keep1;
     }
     __syncthreads();
+}
+
+// ---------------------------------------------------------------------------
+// Fused decode -> GEMM through a ring (kModeGemmTile; speculative runs).
+//
+// What bounds the modes above is X: a round of 512 segments holds two rows of
+// 17408 columns (six of 5120), and X is read from L2 again for every round,
+// 64 bytes of each row of X at a time. Here a round's exponent bytes go to a
+// ring of the workgroup's own in a workspace (a byte a weight, written and
+// read by one CU, so mostly through its L2), and the products are taken once
+// kTileRows whole rows of W are there: X is read once per 16 rows, 256
+// contiguous bytes of each of its rows at a time, and a sign/mantissa byte
+// and an exponent byte of W once, 128 contiguous bytes (a cache line) of each
+// row. The order of a contraction's terms is free: MFMA m of a slice of 128
+// columns takes columns 32 q + 8 m .. + 7 of it in lane quarter q, so a lane
+// reads 32 contiguous bytes of exponents and of sign/mantissa for four MFMAs.
+//
+// A workgroup's first and last row may be shared with its neighbours. A tile
+// that holds such a row takes its columns in up to three intervals, each with
+// its own set of whole rows; a row's sums of an interval it has no weights in
+// are dropped, not multiplied by zero, so an infinite X makes no NaN.
+//
+// The waves split a tile's slices of kSliceCols columns; with fewer slices
+// than waves, several tiles are taken at a time. A wave loads a slice in
+// memory order (8 lanes to a row's 128 bytes of exponents or sign/mantissa)
+// and passes it as bf16 through its own piece of LDS into the MFMA's lane
+// layout: loads straight into that layout put 16 rows in 16 consecutive
+// lanes, and the address unit then takes a cache line a lane (127 us against
+// 103 on the layer below). X comes packed in that layout (pack_x_kernel, one
+// small launch before, which also clears y in the place of a fill).
+//
+// Measured (one box, 65536-symbol chunks unless said, before: the modes
+// above): 5120x17408 with 16 rows of x 332 -> 100 us (97 at 1024-symbol
+// chunks), with 5 rows 228 -> 95; the 151936x5120 head at 1024-symbol chunks
+// with 8 rows 964 -> 684 us. What bounds it now: without the products the
+// layer takes 65 us and the head 472; the exponents are written once and read
+// once more past the L2 (82 KB a workgroup at 5120 columns, 64 workgroups an
+// L2 of 4 MB), so the memory traffic is the bf16 decode's, and a workgroup
+// that waits for it leaves its CU to one decoding workgroup. Tiles of 8 or 4
+// rows, which the L2 would hold, cost more in passes (115 and 128 us); so did
+// a first tile cut short in half of the workgroups, to put their passes at
+// different times (109).
+// ---------------------------------------------------------------------------
+
+constexpr uint32_t kTileRows = 16;
+constexpr uint32_t kSliceCols = 128;
+// The most elements a round adds to the ring.
+constexpr uint32_t kRingRound = kThreads * kSlotCap + 16;
+constexpr uint32_t kSliceBytes = 2 * kTileRows * kSliceCols;  // a wave's piece of LDS (bf16)
+static_assert(kSliceBytes >= 64 * 16, "a wave's sums fit its piece");
+
+// Where column group u (8 columns) of a row stands in a wave's piece: the
+// groups are permuted within the row, so that the rows that one read (the
+// same group of 16 rows) or one write (every second group of 4 rows) meets
+// fall in different banks.
+__device__ __forceinline__ uint32_t slice_at(uint32_t row, uint32_t u) {
+    return row * (2 * kSliceCols) + 16u * (u ^ row);
+}
+
+// Order for LDS that one wave's lanes write and other lanes of it read: the
+// LDS takes a wave's instructions in order, so only the compiler is held back.
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// Column groups of packed X: whole slices.
+__host__ __device__ __forceinline__ constexpr uint32_t x_groups(uint32_t cols) {
+    return (cols + kSliceCols - 1) / kSliceCols * (kSliceCols / 8);
+}
+
+// Where the workgroup's elements stand in the ring.
+struct Ring {
+    uint8_t* base;
+    uint32_t nbytes;    // ring rows * cols
+    uint32_t rows;      // ring rows
+    uint32_t at;        // ring byte of the next element to write
+    uint32_t row;       // first row of W whose products are not taken yet
+    uint32_t row_slot;  // its ring row
+    uint32_t c_head;    // the first column of it that the workgroup holds
+};
+
+__device__ __forceinline__ Ring ring_init(const GemvArgs& G, uint32_t a0) {
+    Ring R;
+    R.rows = G.ring_rows;
+    R.nbytes = G.ring_rows * G.cols;
+    R.base = G.ring + static_cast<uint64_t>(blockIdx.x) * R.nbytes;
+    R.row = a0 / G.cols;
+    R.row_slot = 0;
+    R.c_head = a0 - R.row * G.cols;
+    R.at = R.c_head;
+    return R;
+}
+
+// Groups [0, nfull) of a staged round to the ring.
+__device__ __forceinline__ void ring_put(Ring& R, const uint8_t* stage, uint32_t nfull, uint32_t tid) {
+    uint2 ev[kStoreBatch];
+#pragma unroll
+    for (uint32_t k = 0; k < kStoreBatch; ++k)
+        ev[k] = *reinterpret_cast<const uint2*>(stage + (k * kThreads + tid) * 8);
+#pragma unroll
+    for (uint32_t k = 0; k < kStoreBatch; ++k) {
+        const uint32_t v = k * kThreads + tid;
+        uint32_t p = R.at + 8 * v;
+        p = p >= R.nbytes ? p - R.nbytes : p;
+        if (v < nfull) *reinterpret_cast<uint2*>(R.base + p) = ev[k];
+    }
+    R.at += 8 * nfull;
+    if (R.at >= R.nbytes) R.at -= R.nbytes;
+}
+
+// X for ring_products, and Y's first value. packed: for each 32 columns and
+// each quarter q of them, column group q of every row of X (16 bytes a row),
+// zero past the columns; y (when zero_y) is cleared.
+__global__ __launch_bounds__(256) void pack_x_kernel(const uint16_t* x, uint32_t nb, uint32_t cols,
+                                                     uint32_t n_groups, uint16_t* packed, float* y,
+                                                     int64_t n_y) {
+    const uint32_t stride = gridDim.x * blockDim.x;
+    const uint32_t t0 = blockIdx.x * blockDim.x + threadIdx.x;
+    for (uint32_t p = t0; p < n_groups * nb; p += stride) {
+        const uint32_t g = p / nb, row = p - g * nb;
+        uint4 v = make_uint4(0u, 0u, 0u, 0u);
+        if (8 * g < cols) v = *reinterpret_cast<const uint4*>(x + static_cast<uint64_t>(row) * cols + 8 * g);
+        reinterpret_cast<uint4*>(packed)[p] = v;
+    }
+    for (int64_t k = t0; k < n_y; k += stride) y[k] = 0.0f;
+}
+
+// What a lane loads of a slice: exponents and sign/mantissa bytes of 16
+// columns of two rows of W, four MFMA operands of X.
+struct TileFrag {
+    v4u32 e[2], sm[2], x[4];
+};
+
+__device__ __forceinline__ void consume(const TileFrag& F) {
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) {
+        consume(F.sm[0][k]);
+        consume(F.e[0][k]);
+        consume(F.sm[1][k]);
+        consume(F.e[1][k]);
+#pragma unroll
+        for (uint32_t m = 0; m < 4; ++m) consume(F.x[m][k]);
+    }
+}
+
+// The products of rows R.row .. + nrows - 1 (in the ring; the last one up to
+// column c_tail) with X, added to Y. Every thread calls it, with the ring's
+// writes and every stage read before a barrier; `area` (kWaves * kSliceBytes
+// of LDS) is free. Ends with a barrier.
+__device__ __forceinline__ void ring_products(Ring& R, const DevTensor& T, const GemvArgs& G,
+                                              uint32_t nrows, uint32_t c_tail, uint32_t tid,
+                                              uint8_t* area) {
+    const uint32_t cols = G.cols;
+    const uint32_t nb = static_cast<uint32_t>(G.batch);
+    const uint32_t lane = tid & 63u, w = uniform(tid >> 6);
+    const __amdgpu_buffer_rsrc_t er = buffer_of(R.base, R.nbytes);
+    const __amdgpu_buffer_rsrc_t sr = buffer_of(T.sm, static_cast<uint32_t>(T.n_symbols));
+    const __amdgpu_buffer_rsrc_t xr = buffer_of(G.x, x_groups(cols) * nb * 16u);
+    // Waves a tile, tiles at a time.
+    const uint32_t lg_w = cols > 4 * kSliceCols ? 3u : cols > 2 * kSliceCols ? 2u : cols > kSliceCols ? 1u : 0u;
+    const uint32_t n_at = static_cast<uint32_t>(kWaves) >> lg_w;
+    const uint32_t w_in = w & ((1u << lg_w) - 1u), t_in = w >> lg_w;
+    // The lane's place in a load of W: rows lr and lr + 8, columns 16 lp .. +
+    // 15; and in the MFMA: row r (of W and of X), lane quarter q.
+    const uint32_t lr = lane >> 3, lp = lane & 7u;
+    const uint32_t r = lane & 15u, q = lane >> 4;
+    const uint32_t xo = r < nb ? (q * nb + r) * 16u : 0x80000000u;
+    uint8_t* const mine = area + w * kSliceBytes;
+    for (uint32_t i0 = 0; i0 < nrows; i0 += n_at * kTileRows) {
+        const uint32_t i = i0 + t_in * kTileRows;  // the wave's tile: rows i .. i + n_in - 1
+        f32x4_t sum = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        if (i < nrows) {
+            const uint32_t n_in = nrows - i < kTileRows ? nrows - i : kTileRows;
+            // Where the first row's columns begin, and the last row's end.
+            const uint32_t ch = i == 0 ? R.c_head : 0u;
+            const uint32_t ct = i + n_in == nrows ? c_tail : cols;
+            uint32_t eo[2], so[2];
+#pragma unroll
+            for (uint32_t h = 0; h < 2; ++h) {
+                const uint32_t k = lr + 8 * h;
+                uint32_t slot = R.row_slot + i + k;
+                slot = slot >= R.rows ? slot - R.rows : slot;
+                eo[h] = k < n_in ? slot * cols + 16u * lp : 0x80000000u;
+                so[h] = k < n_in ? (R.row + i + k) * cols + 16u * lp : 0x80000000u;
+            }
+            uint32_t lo = 0;
+            while (lo < cols) {
+                // The interval: up to the next of ch, ct and cols.
+                uint32_t hi = cols;
+                if (lo < ch) hi = ch;
+                if (lo < ct && ct < hi) hi = ct;
+                if (n_in == 1 && (lo < ch || lo >= ct)) {  // no row has weights here
+                    lo = hi;
+                    continue;
+                }
+                f32x4_t d = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+                // (Loads past the interval return zero without reading memory:
+                // issued on every path, so that a wait counts the loads of
+                // one slice and not all in flight.)
+                auto issue = [&](TileFrag& F, uint32_t at) {
+                    const uint32_t c = uniform(at < hi ? at : 0u);
+                    const uint32_t out = at < hi ? 0u : 0x80000000u;
+#pragma unroll
+                    for (uint32_t h = 0; h < 2; ++h) {
+                        const auto s = __builtin_amdgcn_raw_buffer_load_b128(sr, so[h] | out, c, 0);
+                        const auto e = __builtin_amdgcn_raw_buffer_load_b128(er, eo[h] | out, c, 0);
+                        F.sm[h] = v4u32{s[0], s[1], s[2], s[3]};
+                        F.e[h] = v4u32{e[0], e[1], e[2], e[3]};
+                    }
+#pragma unroll
+                    for (uint32_t m = 0; m < 4; ++m) {
+                        const auto x = __builtin_amdgcn_raw_buffer_load_b128(xr, xo | out, (c + 32 * m) * 2u * nb, 0);
+                        F.x[m] = v4u32{x[0], x[1], x[2], x[3]};
+                    }
+                };
+                auto multiply = [&](const TileFrag& F, uint32_t c) {
+                    const bool whole = c >= lo && c + kSliceCols <= hi;
+#pragma unroll
+                    for (uint32_t k = 0; k < 4; ++k) {
+                        const uint32_t h = k >> 1, j = 2 * (k & 1u);
+                        const uint2 pa = bf16_quad(F.sm[h][j], F.e[h][j]);
+                        const uint2 pb = bf16_quad(F.sm[h][j + 1], F.e[h][j + 1]);
+                        uint4 wv = make_uint4(pa.x, pa.y, pb.x, pb.y);
+                        if (!whole) {
+                            // Columns outside the interval: neither W (another
+                            // row's, or no weight's, bytes) nor X.
+                            const uint32_t g = c + 16u * lp + 8u * (k & 1u);
+                            wv = g >= lo && g < hi ? wv : make_uint4(0u, 0u, 0u, 0u);
+                        }
+                        *reinterpret_cast<uint4*>(mine + slice_at(lr + 8 * h, 2 * lp + (k & 1u))) = wv;
+                    }
+                    wave_lds_order();
+#pragma unroll
+                    for (uint32_t m = 0; m < 4; ++m) {
+                        const uint4 wv = *reinterpret_cast<const uint4*>(mine + slice_at(r, 4 * m + q));
+                        uint4 xv = make_uint4(F.x[m][0], F.x[m][1], F.x[m][2], F.x[m][3]);
+                        if (!whole) {
+                            const uint32_t g = c + 32u * m + 8u * q;
+                            xv = g >= lo && g < hi ? xv : make_uint4(0u, 0u, 0u, 0u);
+                        }
+                        d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, xv),
+                                                                    __builtin_bit_cast(bf16x8_t, wv), d, 0,
+                                                                    0, 0);
+                    }
+                    wave_lds_order();
+                };
+                // Slices w_in, w_in + waves a tile, ... (One in flight a wave:
+                // two or three at half the width were 2% and 15% slower, as
+                // the registers they take spill.)
+                const uint32_t step = kSliceCols << lg_w;
+                uint32_t c = (lo & ~(kSliceCols - 1u)) + w_in * kSliceCols;
+                TileFrag F;
+                issue(F, c);
+                while (c < hi) {
+                    consume(F);
+                    multiply(F, c);
+                    c += step;
+                    issue(F, c);
+                }
+                const bool has = r < n_in && !(r == 0 && lo < ch) && !(r == n_in - 1 && lo >= ct);
+#pragma unroll
+                for (uint32_t k = 0; k < 4; ++k) sum[k] += has ? d[k] : 0.0f;
+                lo = hi;
+            }
+        }
+        *reinterpret_cast<f32x4_t*>(mine + 16 * lane) = sum;
+        __syncthreads();
+        const uint32_t n_e = n_at * 256;
+        for (uint32_t j = tid; j < n_e; j += kThreads) {
+            // Entry k of lane l2 of the waves of tile j / 256.
+            const uint32_t l2 = (j >> 2) & 63u, k = j & 3u, tj = j >> 8;
+            const uint8_t* const f = area + (tj << lg_w) * kSliceBytes + 4 * (j & 255u);
+            float a = 0.0f;
+            for (uint32_t v = 0; v < (1u << lg_w); ++v) a += *reinterpret_cast<const float*>(f + v * kSliceBytes);
+            const uint32_t t = 4 * (l2 >> 4) + k;
+            const uint32_t ri = i0 + tj * kTileRows + (l2 & 15u);
+            if (t < nb && ri < nrows && a != 0.0f)
+                atomicAdd(G.y + static_cast<int64_t>(t) * G.rows + R.row + ri, a);
+        }
+        __syncthreads();
+    }
+    R.row += nrows;
+    R.row_slot += nrows;
+    if (R.row_slot >= R.rows) R.row_slot -= R.rows;
+    R.c_head = 0;
 }
 
 // Vector groups [0, nfull) of the staged round to output elements a0...;
@@ -3001,6 +3298,7 @@ static_assert(kSpecStageBytes >= kStoreBatch * kThreads * 8, "store batches read
 static_assert(kSpecStageBytes >= kStoreBatch * kThreads * 16 / 2, "u8 store batches too");
 static_assert(kSpecStageBytes >= kGemmRedOffset + kGemmRedBytes, "a GEMM piece and its sums fit the stage");
 static_assert(kSpecStageBytes >= kSpecDense + 16, "the GEMM round keeps the carried bytes");
+static_assert(kSpecStageBytes >= kLeadBytes + kWaves * kSliceBytes, "a ring tile's slices fit the stage");
 // A chunk of this many bytes or more makes its table unusable (the exact
 // fallback decodes it): segment counts come from a multiply-high that is
 // exact below it, and its bit count fits 32 bits.
@@ -3219,7 +3517,7 @@ __device__ void spec_piece(SpecLds& lds, const Tables& tb, bool global_esc, cons
     SpecTab tab = spec_tab_commit(TF, T, lds, b, ca, cb, 0u, 0u, false, S, smagic, lane, w, &jj);
     uint32_t c0 = ca;     // chunk of the round's first segment
     uint32_t p0 = 0;      // chunk bit where its first codeword starts (k0 > 0)
-    GemmAcc gacc;         // fused GEMM: this wave's partial sums
+    GemmAcc gacc;         // fused GEMM without a ring: this wave's partial sums
     gemm_acc_init(gacc);
     uint32_t rank0 = 0;   // codewords of chunk c0 before the round
     uint32_t lead = 0;    // carried symbols at the front of the stage
@@ -3240,6 +3538,8 @@ __device__ void spec_piece(SpecLds& lds, const Tables& tb, bool global_esc, cons
     const IlSlot sl{lds.stage + kLeadBytes, w * kSlotRows * 256u, lane * 4u};
     const int64_t piece_end = static_cast<int64_t>(cb) * cs < T.n_symbols ? static_cast<int64_t>(cb) * cs
                                                                          : T.n_symbols;
+    Ring ring{};
+    if constexpr (kMode == kModeGemmTile) ring = ring_init(args.gemv, static_cast<uint32_t>(a0));
     while (fall_from < 0) {
         const uint32_t ns = tab.ns;
         // The next round (found when this round's table was committed).
@@ -3255,6 +3555,14 @@ __device__ void spec_piece(SpecLds& lds, const Tables& tb, bool global_esc, cons
         }
         SmBatch<kMode> smb;
         sm_issue<kMode, kGroup>(smb, T, a0, tid, kThreads, static_cast<uint32_t>(piece_end));
+        // A word of every 128 bytes of the round's sign/mantissa bytes, so
+        // that they are in a cache when the tile's products read them (layer
+        // 100.4 -> 97.0 us, head 714 -> 684).
+        uint32_t sm_touch = 0;
+        if constexpr (kMode == kModeGemmTile)
+            sm_touch = __builtin_amdgcn_raw_buffer_load_b32(
+                buffer_of(T.sm, static_cast<uint32_t>(piece_end)),
+                (static_cast<uint32_t>(a0) & ~3u) + (tid < kRingRound / 128 ? 128u * tid : 0x80000000u), 0, 0);
 
         // Chunk c0's output count and the stage's first place in it.
         const uint32_t lim0 = static_cast<uint32_t>(
@@ -3384,6 +3692,7 @@ __device__ void spec_piece(SpecLds& lds, const Tables& tb, bool global_esc, cons
             tabn = spec_tab_commit(TF, T, lds, b ^ 1u, c0n, cb, k0n, offn, true, S, smagic, lane, w,
                                    &jjn);
         }
+        if constexpr (kMode == kModeGemmTile) consume(sm_touch);
         __syncthreads();  // B: slots read; the next table and words written
         const bool bad_round = lds.bad != 0u;
         const uint32_t avail = uniform(lds.last[2]);
@@ -3409,15 +3718,20 @@ __device__ void spec_piece(SpecLds& lds, const Tables& tb, bool global_esc, cons
         __syncthreads();  // C: the round's symbols are in place
         if (bad_round) {
             fall_from = a0;
-            break;
+            if constexpr (kMode != kModeGemmTile) break;
         }
         // Whole vector groups, never past the piece's end.
         const int64_t room = (piece_end - a0) / kGroup;
         const uint32_t nfull0 = avail / kGroup;
-        const uint32_t nfull = room < static_cast<int64_t>(nfull0) ? static_cast<uint32_t>(room > 0 ? room : 0)
-                                                                  : nfull0;
+        uint32_t nfull = room < static_cast<int64_t>(nfull0) ? static_cast<uint32_t>(room > 0 ? room : 0)
+                                                            : nfull0;
         __builtin_amdgcn_s_setprio(2);
-        store_round<kMode, kGroup, true>(smb, T, args.gemv, stage, a0, nfull, tid, kThreads, 0, &gacc);
+        if constexpr (kMode == kModeGemmTile) {
+            if (bad_round) nfull = 0;
+            ring_put(ring, stage, nfull, tid);
+        } else {
+            store_round<kMode, kGroup, true>(smb, T, args.gemv, stage, a0, nfull, tid, kThreads, 0, &gacc);
+        }
         // The partial vector group moves to the front.
         const uint32_t rem0 = avail - nfull * kGroup;
         const uint32_t rem = rem0 < static_cast<uint32_t>(kGroup) ? rem0 : kGroup - 1u;
@@ -3435,6 +3749,21 @@ __device__ void spec_piece(SpecLds& lds, const Tables& tb, bool global_esc, cons
         }
         a0 += static_cast<int64_t>(nfull) * kGroup;
         lead = rem;
+        if constexpr (kMode == kModeGemmTile) {
+            // Products of the whole tiles in the ring; of everything in it
+            // when no round follows.
+            const bool last = !more || bad_round || tabn.bad != 0u;
+            const uint32_t end = uniform(static_cast<uint32_t>(a0));
+            const uint32_t er = end / args.gemv.cols;
+            const uint32_t ec = end - er * args.gemv.cols;
+            const uint32_t have = er - ring.row;
+            const uint32_t nrows = last ? have + (ec != 0 ? 1u : 0u) : have / kTileRows * kTileRows;
+            const bool any = last ? end > ring.row * args.gemv.cols + ring.c_head : nrows != 0;
+            if (any)
+                ring_products(ring, T, args.gemv, nrows, last && ec != 0 ? ec : args.gemv.cols, tid,
+                              stage + kLeadBytes);
+            if (bad_round) break;
+        }
         if (!more) break;
         if (tabn.bad != 0u) {
             fall_from = a0;
@@ -3458,7 +3787,7 @@ __device__ void spec_piece(SpecLds& lds, const Tables& tb, bool global_esc, cons
         // codeword (exact on any input).
         run_fallback<kMode>(tb, args, T, fall_from / cs, cb, fall_from);
     }
-    if constexpr (is_gemm(kMode)) gemm_finish(gacc, args.gemv, stage);
+    if constexpr (keeps_tile_sums(kMode)) gemm_finish(gacc, args.gemv, stage);
     __syncthreads();  // LDS is free for the next piece
 }
 
@@ -3766,6 +4095,13 @@ int launch_batch(Batch& B, hipStream_t s, bool tiny) {
     return AIMG_OK;
 }
 
+int fail_gemm_layout() {
+    return fail(AIMG_ERR_UNSUPPORTED,
+                "fused GEMM: needs chunk_size a multiple of 8 and >= " + std::to_string(kRunMinChunk) +
+                    ", at most 2^24, 8-byte aligned sign_mantissa, 4 or more packed bytes and below "
+                    "4 GiB - 1 MiB");
+}
+
 // Validate tensor i and add it to the normal or the tiny-buffer batch.
 // The segment-run kernel over the batch's tensors: a full grid, whose
 // workgroups split the tensors' segments evenly among themselves.
@@ -3907,6 +4243,63 @@ int add_tensor(const aimg_tensor& t, int i, Batch& normal, Batch& tiny, Batch* r
     return AIMG_OK;
 }
 
+// The checks of launch() on one tensor of a fused GEMM, without the launch.
+template <int kMode>
+int check_tensor(const aimg_tensor& t) {
+    Batch normal, tiny, spec;
+    const int rc = add_tensor<kMode>(t, 0, normal, tiny, nullptr, &spec, true);
+    if (rc != AIMG_OK) return rc;
+    return normal.m == 0 && tiny.m == 0 ? AIMG_OK : fail_gemm_layout();
+}
+
+// Whether the ring serves an n_x-row GEMM faster than the modes without it
+// (microseconds without, with; 1024-symbol chunks unless said). Rows of more
+// than kGemmPieceMaxCols columns: always (4x20480, 16 rows of x: 37, 18;
+// 3000x20480: 249, 77). Shorter ones: X is read once a piece of 2048 groups
+// without the ring, which costs more with more rows of x and more columns.
+// 16 rows: 30000x1000 43, 48; 30000x1400 61, 59; 8000x2048 36, 32; 800x5120
+// 26, 23. 5 rows: 8000x2048 31, 32; 30000x2048 71, 70; 800x5120 21, 23;
+// 2000x4096 26, 25; 4096x4096 at 65536 symbols 38, 32. n_x 0: not asked.
+bool ring_pays(int64_t n_symbols, int64_t cols, int n_x) {
+    if (n_x == 0 || cols > kGemmPieceMaxCols) return true;
+    if (n_x > 8) return cols >= 2048;
+    return cols >= 4096 && n_symbols >= (int64_t{1} << 23);
+}
+
+// Rows of a workgroup's ring for a rows x cols weight in chunks of
+// chunk_size, and the workgroups of its launch (kModeGemmTile): room for a
+// tile whose last row is one element short and the round that completes it,
+// or for everything a workgroup can be given, if that is less. 0 rows: no
+// ring (the total would pass kRingMaxBytes, or a 32-bit offset would not do).
+constexpr int64_t kRingMaxBytes = int64_t{512} << 20;
+
+struct RingPlan {
+    int64_t rows = 0;
+    int64_t grid = 0;
+    int64_t x_at = 0;   // workspace byte of packed X (after the rings)
+    size_t nbytes = 0;  // of the workspace; 0: no ring
+};
+
+RingPlan plan_ring(int64_t n_symbols, int64_t cols, int64_t chunk_size) {
+    RingPlan P;
+    const int64_t slots = static_cast<int64_t>(cu_count()) * kBlocksPerCu;
+    const int64_t chunks = (n_symbols + chunk_size - 1) / chunk_size;
+    P.grid = chunks < slots ? chunks : slots;
+    if (P.grid < 1) return P;
+    // (launch_spec: a workgroup's chunks are at most a CU's share, rounded up.)
+    const int64_t cus = P.grid == slots && slots % 2 == 0 ? slots / 2 : P.grid;
+    const int64_t share = (chunks / cus + 2) * chunk_size;
+    const int64_t need = kTileRows + (kRingRound + cols - 1) / cols;
+    const int64_t all = (share < n_symbols ? share : n_symbols) / cols + 2;
+    const int64_t rows = need < all ? need : all;
+    if (rows * cols >= (int64_t{1} << 30) || kTileRows * cols * 2 >= (int64_t{1} << 30)) return P;
+    if (rows * cols * P.grid > kRingMaxBytes) return P;
+    P.rows = rows;
+    P.x_at = (rows * cols * P.grid + 255) / 256 * 256;
+    P.nbytes = static_cast<size_t>(P.x_at) + size_t{16} * kGemmMaxRows * x_groups(static_cast<uint32_t>(cols));
+    return P;
+}
+
 // vec_ok false selects the element-wise kernel whatever the tensors' layout.
 template <int kMode>
 int launch(const aimg_tensor* ts, int n, const GemvArgs& gemv, bool vec_ok, void* stream) {
@@ -3940,11 +4333,7 @@ int launch(const aimg_tensor* ts, int n, const GemvArgs& gemv, bool vec_ok, void
             const int rc = add_tensor<kMode>(ts[i], i, normal, tiny, nullptr, vec_ok ? &spec : nullptr, true);
             if (rc != AIMG_OK) return rc;
         }
-        if (normal.m != 0 || tiny.m != 0)
-            return fail(AIMG_ERR_UNSUPPORTED,
-                        "fused GEMM: needs chunk_size a multiple of 8 and >= " + std::to_string(kRunMinChunk) +
-                            ", at most 2^24, 8-byte aligned sign_mantissa, 4 or more packed bytes and below "
-                            "4 GiB - 1 MiB");
+        if (normal.m != 0 || tiny.m != 0) return fail_gemm_layout();
         return launch_spec<kMode>(spec, s);
     } else {
     Batch* const to_run = vec_ok && !no_runs ? &run : nullptr;
@@ -4122,7 +4511,7 @@ extern "C" int aimg_decode_gemv_bf16(const aimg_tensor* t, int64_t rows, int64_t
     const uint32_t step = aimg::kThreads * 8;  // elements between a thread's groups
     const aimg::GemvArgs g{static_cast<const uint16_t*>(x), y, static_cast<uint32_t>(rows),
                            static_cast<uint32_t>(cols), batch,
-                           step / static_cast<uint32_t>(cols), step % static_cast<uint32_t>(cols)};
+                           step / static_cast<uint32_t>(cols), step % static_cast<uint32_t>(cols), nullptr, 0u};
     // The 8-weight groups take 16-byte x loads: they must lie inside one row
     // (cols % 8 == 0) and x must be 16-byte aligned.
     const bool vec_ok = cols % 8 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0;
@@ -4130,8 +4519,11 @@ extern "C" int aimg_decode_gemv_bf16(const aimg_tensor* t, int64_t rows, int64_t
     return aimg::launch<aimg::kModeGemv>(t, 1, g, vec_ok, stream);
 }
 
-extern "C" int aimg_decode_gemm_bf16(const aimg_tensor* t, int64_t rows, int64_t cols,
-                                     const void* x, int n_x, float* y, void* stream) {
+namespace {
+
+// Arguments of the fused GEMM, checked; x with a row stride and alignment it
+// does not take is refused.
+int check_gemm(const aimg_tensor* t, int64_t rows, int64_t cols, const void* x, int n_x, const float* y) {
     using aimg::fail;
     if (t == nullptr) return fail(AIMG_ERR_INVALID_ARGUMENT, "tensor is null");
     if (rows < 1 || cols < 1 || rows > INT32_MAX || cols > INT32_MAX ||
@@ -4144,8 +4536,64 @@ extern "C" int aimg_decode_gemm_bf16(const aimg_tensor* t, int64_t rows, int64_t
         static_cast<int64_t>(n_x) * cols * 2 > int64_t{0xFFFFFFFF})
         return fail(AIMG_ERR_UNSUPPORTED,
                     "fused GEMM: needs cols % 8 == 0, a 16-byte aligned x and n_x * cols * 2 below 2^32");
+    return AIMG_OK;
+}
+
+}  // namespace
+
+extern "C" int aimg_decode_gemm_bf16(const aimg_tensor* t, int64_t rows, int64_t cols,
+                                     const void* x, int n_x, float* y, void* stream) {
+    const int rc = check_gemm(t, rows, cols, x, n_x, y);
+    if (rc != AIMG_OK) return rc;
     const aimg::GemvArgs g{static_cast<const uint16_t*>(x), y, static_cast<uint32_t>(rows),
-                           static_cast<uint32_t>(cols), n_x, 0u, 0u};
+                           static_cast<uint32_t>(cols), n_x, 0u, 0u, nullptr, 0u};
     if (cols > aimg::kGemmPieceMaxCols) return aimg::launch<aimg::kModeGemmRows>(t, 1, g, true, stream);
     return aimg::launch<aimg::kModeGemm>(t, 1, g, true, stream);
+}
+
+extern "C" int aimg_gemm_workspace_nbytes(const aimg_tensor* t, int64_t rows, int64_t cols, int n_x,
+                                          size_t* nbytes) {
+    using aimg::fail;
+    if (t == nullptr || nbytes == nullptr) return fail(AIMG_ERR_INVALID_ARGUMENT, "null tensor or nbytes");
+    if (rows < 1 || cols < 1 || rows > INT32_MAX || cols > INT32_MAX || rows * cols != t->n_symbols)
+        return fail(AIMG_ERR_INVALID_ARGUMENT, "rows * cols must equal n_symbols (both >= 1)");
+    if (n_x < 0 || n_x > aimg::kGemmMaxRows)
+        return fail(AIMG_ERR_INVALID_ARGUMENT, "n_x must be in 0.." + std::to_string(aimg::kGemmMaxRows));
+    *nbytes = 0;
+    if (cols % 8 != 0 || t->chunk_size < 8 || !aimg::ring_pays(t->n_symbols, cols, n_x)) return AIMG_OK;
+    *nbytes = aimg::plan_ring(t->n_symbols, cols, t->chunk_size).nbytes;
+    return AIMG_OK;
+}
+
+extern "C" int aimg_decode_gemm_bf16_ws(const aimg_tensor* t, int64_t rows, int64_t cols, const void* x,
+                                        int n_x, float* y, int zero_y, void* workspace,
+                                        size_t workspace_nbytes, void* stream) {
+    using aimg::fail;
+    int rc = check_gemm(t, rows, cols, x, n_x, y);
+    if (rc != AIMG_OK) return rc;
+    const aimg::RingPlan P = aimg::plan_ring(t->n_symbols, cols, t->chunk_size < 1 ? 1 : t->chunk_size);
+    if (P.nbytes == 0 || workspace == nullptr || workspace_nbytes < P.nbytes ||
+        reinterpret_cast<uintptr_t>(workspace) % 16 != 0)
+        return fail(AIMG_ERR_INVALID_ARGUMENT,
+                    "the workspace is null, misaligned or below aimg_gemm_workspace_nbytes");
+    uint8_t* const ws = static_cast<uint8_t*>(workspace);
+    uint16_t* const packed = reinterpret_cast<uint16_t*>(ws + P.x_at);
+    const aimg::GemvArgs g{packed, y, static_cast<uint32_t>(rows), static_cast<uint32_t>(cols), n_x, 0u, 0u,
+                           ws, static_cast<uint32_t>(P.rows)};
+    // X into its packed layout (and y cleared) before the decode; a refused
+    // tensor is refused before anything is launched.
+    rc = aimg::check_tensor<aimg::kModeGemmTile>(*t);
+    if (rc != AIMG_OK) return rc;
+    const uint32_t xg = aimg::x_groups(static_cast<uint32_t>(cols));
+    const int64_t n_y = zero_y ? static_cast<int64_t>(n_x) * rows : 0;
+    const int64_t work = n_y > static_cast<int64_t>(xg) * n_x ? n_y : static_cast<int64_t>(xg) * n_x;
+    const int64_t cap = static_cast<int64_t>(aimg::cu_count()) * 8;
+    const int64_t want = (work + 255) / 256;
+    hipLaunchKernelGGL(aimg::pack_x_kernel, dim3(static_cast<uint32_t>(want < cap ? want : cap)), dim3(256), 0,
+                       static_cast<hipStream_t>(stream), static_cast<const uint16_t*>(x),
+                       static_cast<uint32_t>(n_x), static_cast<uint32_t>(cols), xg, packed, y, n_y);
+    const hipError_t err = hipGetLastError();
+    if (err != hipSuccess)
+        return fail(AIMG_ERR_HIP, std::string("kernel launch failed: ") + hipGetErrorString(err));
+    return aimg::launch<aimg::kModeGemmTile>(t, 1, g, true, stream);
 }

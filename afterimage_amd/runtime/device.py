@@ -542,7 +542,8 @@ def decode_gemm(t: DeviceTensor, x: torch.Tensor, rows: int, cols: int,
                 y: torch.Tensor | None = None) -> torch.Tensor:
     """decode_gemv for 1..GEMM_MAX_ROWS rows of x (speculative-verify
     widths), on the matrix cores: bf16 products, fp32 sums, W decoded inside
-    the kernel and never written. Needs cols % 8 == 0 and chunks of 1024 to
+    the kernel and never written (long rows: a tile's exponents at a time pass
+    through scratch memory from torch's allocator). Needs cols % 8 == 0 and chunks of 1024 to
     2^24 symbols (a multiple of 8); other layers raise (the blocked
     decode_linear serves them)."""
     return _fused(t, x, rows, cols, y, GEMM_MAX_ROWS, "aimg_decode_gemm_bf16")
@@ -560,20 +561,45 @@ def _fused(t: DeviceTensor, x: torch.Tensor, rows: int, cols: int, y: torch.Tens
         raise ValueError("batch must be in 1..%d, got %d" % (max_b, b))
     if rows * cols != t.n_symbols:
         raise ValueError("rows * cols = %d, the tensor has %d weights" % (rows * cols, t.n_symbols))
-    if y is None:
-        y = torch.zeros((b, rows), dtype=torch.float32, device=dev)
-    elif y.dtype != torch.float32 or tuple(y.shape) != (b, rows) or not y.is_contiguous():
+    if y is not None and (y.dtype != torch.float32 or tuple(y.shape) != (b, rows) or not y.is_contiguous()):
         raise ValueError("y must be a contiguous fp32 [%d, %d] tensor" % (b, rows))
     if t.sign_mantissa is None or t.sign_mantissa.device != dev:
         raise ValueError("the tensor needs sign_mantissa bytes on %s" % dev)
-    _check_device(t, y)
+    _check_device(t, x if y is None else y)
     d = (_native.AimgTensor * 1)()
-    d[0] = _descriptor(t, y, t.n_symbols)
-    d[0].out = None
+    d[0] = _descriptor(t, None, t.n_symbols)
     with torch.cuda.device(dev):
-        _native.check(getattr(_native.lib(), entry)(
-            d, rows, cols, x.data_ptr(), b, y.data_ptr(), _stream_handle(dev)))
+        ws = None
+        if entry == "aimg_decode_gemm_bf16" and cols >= 2048:  # (shorter rows take none)
+            ws = _gemm_workspace(d, rows, cols, b, dev)
+        if ws is not None:
+            zero_y = y is None
+            if zero_y:
+                y = torch.empty((b, rows), dtype=torch.float32, device=dev)
+            _native.check(_native.lib().aimg_decode_gemm_bf16_ws(
+                d, rows, cols, x.data_ptr(), b, y.data_ptr(), int(zero_y), ws.data_ptr(), ws.numel(),
+                _stream_handle(dev)))
+        else:
+            if y is None:
+                y = torch.zeros((b, rows), dtype=torch.float32, device=dev)
+            _native.check(getattr(_native.lib(), entry)(
+                d, rows, cols, x.data_ptr(), b, y.data_ptr(), _stream_handle(dev)))
     return y
+
+
+def _gemm_workspace(d, rows: int, cols: int, b: int, dev) -> torch.Tensor | None:
+    """Scratch memory of one fused GEMM, from torch's caching allocator on the
+    current stream (which the launch uses, so the block goes back to the
+    allocator in stream order); None where the shape takes none or the memory
+    is not to be had (the GEMM then runs without it, slower)."""
+    nbytes = ctypes.c_size_t(0)
+    _native.check(_native.lib().aimg_gemm_workspace_nbytes(d, rows, cols, b, ctypes.byref(nbytes)))
+    if nbytes.value == 0:
+        return None
+    try:
+        return torch.empty(nbytes.value, dtype=torch.uint8, device=dev)
+    except torch.OutOfMemoryError:
+        return None
 
 
 def row_blocks(rows: int, cols: int, chunk_size: int, n_chunks: int, slice_rows: int):

@@ -251,6 +251,7 @@ inline void __builtin_amdgcn_s_setprio(int) {}  // wave issue priority: no effec
 // A wave's short sleep: blocks run one after another here, so a wait for a
 // later block only passes its poll count.
 inline void __builtin_amdgcn_s_sleep(int) { std::this_thread::yield(); }
+inline void __builtin_amdgcn_wave_barrier() { emu::g_block->wave[threadIdx.x >> 6]->arrive_and_wait(); }
 inline void __builtin_amdgcn_fence(int, const char*) { __atomic_thread_fence(__ATOMIC_SEQ_CST); }
 #ifndef __HIP_MEMORY_SCOPE_AGENT
 #define __HIP_MEMORY_SCOPE_AGENT 4

@@ -127,3 +127,42 @@ def test_rejects_what_it_does_not_serve():
     # The blocked path serves the same layer.
     y = decompress_linear_gpu(small, x.reshape(1, 6, 256))
     _check(y.reshape(6, 40), _ref(W, x))
+
+
+def _ring_bound(W, x):
+    """|fp32 sum of exact bf16 products - exact| <= cols * 2^-24 * sum |w x|
+    for any order of the additions (one rounding a term)."""
+    return W.shape[1] * 2.0 ** -24 * (x.double().abs() @ W.double().abs().t()) + 1e-30
+
+
+@pytest.mark.parametrize("shape,chunk,n_x", [((31, 18000), 5000, 12), ((4, 20480), 1024, 16),
+                                             ((1, 8200), 65536, 1), ((700, 2056), 1024, 9),
+                                             ((2100, 4104), 8192, 5), ((5120, 2048), 1000 + 24, 16),
+                                             ((257, 9000), 2048, 3)])
+def test_ring(shape, chunk, n_x):
+    """The GEMM through a ring in a workspace: workgroups that begin and end
+    inside a row, rows of more than one round, a last 128-column slice cut
+    short, fewer rows than a tile."""
+    W = workloads.bf16_normal(shape, 80 + n_x, 0.02, outlier_frac=1e-3)
+    layer = compress_layer(W, chunk_size=chunk)
+    x = _x(n_x, shape[1], 5)
+    t = DeviceTensor.from_encoded(layer.encoded, layer.sign_mantissa, "cuda")
+    for _ in range(2):  # the second call finds the first one's workspace
+        y = decode_gemm(t, x.cuda(), *shape).cpu().double()
+        assert bool(((y - x.double() @ W.double().t()).abs() <= _ring_bound(W, x)).all())
+
+
+def test_ring_infinite_x():
+    """An infinite x makes the sums of every row infinite (no NaN: the
+    weights of its column are not zero), also of rows that two workgroups
+    share."""
+    W = workloads.bf16_normal((64, 10000), 9, 0.02)
+    col = 4321
+    W[:, col] = W[:, col].abs() + 0.01
+    layer = compress_layer(W, chunk_size=1024)
+    x = _x(6, 10000, 2)
+    x[2, col] = float("inf")
+    t = DeviceTensor.from_encoded(layer.encoded, layer.sign_mantissa, "cuda")
+    y = decode_gemm(t, x.cuda(), 64, 10000).cpu()
+    assert bool(torch.isposinf(y[2]).all())
+    assert bool(torch.isfinite(y[[0, 1, 3, 4, 5]]).all())

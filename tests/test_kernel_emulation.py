@@ -587,3 +587,22 @@ def test_spec_runs_chunks_out_of_order_and_empty(emu):
 def test_fused_gemm(emu, rows, cols, chunk, n_x):
     _gemv(emu, "gemm_%d_%d_%d_%d" % (rows, cols, chunk, n_x), rows, cols, chunk, n_x, 40 + n_x,
           cus=2, mode="gemm")
+
+
+# The fused GEMM through a ring in a workspace: workgroups that start and end
+# inside a row (chunks that do not divide one), several tiles at a time (rows
+# of one, two and four slices of 128 columns), a last slice cut short, a ring
+# that wraps (many rows a workgroup, one CU), and 64Ki-symbol chunks.
+
+@pytest.mark.parametrize("rows,cols,chunk,n_x,cus", [
+    (300, 200, 1024, 8, 2),
+    (520, 264, 1024, 5, 1),
+    (200, 512, 1000 + 24, 16, 1),
+    (150, 1032, 2048, 1, 1),
+    (40, 5120, 4096, 16, 1),
+    (9, 17408, 65536, 6, 2),
+    (3, 8, 1024, 16, 2),
+])
+def test_fused_gemm_ring(emu, rows, cols, chunk, n_x, cus):
+    _gemv(emu, "ring_%d_%d_%d_%d" % (rows, cols, chunk, n_x), rows, cols, chunk, n_x, 40 + n_x,
+          cus=cus, mode="gemm-ring")
