@@ -178,8 +178,7 @@ struct GemvArgs {
     uint32_t ring_rows;
 };
 
-struct LaunchArgs {
-    DevTensor t[AIMG_MAX_TENSORS];
+struct LaunchHead {
     int64_t total_items;  // speculative runs: the tensors' elements
     int32_t n_tensors;
     // Segment runs: workgroup w takes rounds w, w + grid, ... Speculative
@@ -201,6 +200,30 @@ struct LaunchArgs {
     // second half of the grid starts later.
     int32_t stagger;
 };
+
+// A launch of up to kN tensors. Most launches hold one: most kernels then take
+// that one's 112 bytes instead of the 3.6 KB of AIMG_MAX_TENSORS, which the
+// host copies and the GPU fetches for each launch (1024x3072 bf16 12.8 -> 12.1
+// us, 3001x4099 exponent bytes at 512-symbol chunks 21.7 -> 20.4, 5120x17408
+// GEMM of 16 rows 99.4 -> 97.2, the layer with its index 55.7 -> 54.7).
+template <int kN>
+struct TensorArgs {
+    DevTensor t[kN];
+};
+
+template <int kN>
+struct LaunchArgsN : TensorArgs<kN>, LaunchHead {
+    static constexpr bool kOne = kN == 1;
+    template <typename I>
+    __device__ __forceinline__ const DevTensor& tensor(I d) const {
+        if constexpr (kOne)
+            return this->t[0];
+        else
+            return this->t[d];
+    }
+    __device__ __forceinline__ int count() const { return kOne ? 1 : n_tensors; }
+};
+using LaunchArgs = LaunchArgsN<AIMG_MAX_TENSORS>;
 
 // Read-only launch data that every thread of a workgroup reads at the same
 // address (table header, a workgroup's own chunk offset and length): loaded
@@ -673,8 +696,8 @@ __device__ __forceinline__ bool index_build_ready(const DevTensor& T) {
 }
 
 // kLg > 0: every tensor of the launch has 1 << kLg threads per chunk.
-template <int kMode, uint32_t kLg>
-__device__ __forceinline__ Job make_job(const LaunchArgs& args, int64_t item, uint32_t tid) {
+template <int kMode, uint32_t kLg, class Args>
+__device__ __forceinline__ Job make_job(const Args& args, int64_t item, uint32_t tid) {
     Job J{-1, 0u, kMaxSegBits, 0, 0u, 0u, 0u, 0u, kNoIndex, 0u, 0u, kWholeChunk, 0u};
     if (item >= args.total_items) return J;
     // Split chunk k (chunk item split_first + k): its first half is item k,
@@ -694,8 +717,9 @@ __device__ __forceinline__ Job make_job(const LaunchArgs& args, int64_t item, ui
         }
     }
     int d = 0;
-    while (d + 1 < args.n_tensors && item >= args.t[d + 1].item_begin) ++d;
-    const DevTensor& T = args.t[d];
+    if constexpr (!Args::kOne)
+        while (d + 1 < args.n_tensors && item >= args.t[d + 1].item_begin) ++d;
+    const DevTensor& T = args.tensor(d);
     J.d = d;
     J.lg = kLg > 0 ? kLg : static_cast<uint32_t>(__ffs(T.tpc) - 1);
     const uint32_t n_groups = kThreads >> J.lg;
@@ -799,11 +823,11 @@ __device__ __forceinline__ uint32_t last_word(const DevTensor& T) {
 // byte by byte. Such tensors go to a kernel of their own, which keeps these
 // loads and their waits out of every other kernel's round loop.
 // kLg: threads per chunk as the kernel's (0: the job's own).
-template <int kMode, bool kTiny, uint32_t kLg>
-__device__ __forceinline__ void fetch_issue(Fetch& F, const LaunchArgs& args, const Job& J,
+template <int kMode, bool kTiny, uint32_t kLg, class Args>
+__device__ __forceinline__ void fetch_issue(Fetch& F, const Args& args, const Job& J,
                                             uint32_t r, uint32_t tid) {
     if (round_len(J, r) == 0) return;
-    const DevTensor& T = args.t[J.d];
+    const DevTensor& T = args.tensor(J.d);
     const uint32_t lg = kLg > 0 ? kLg : J.lg;
     const uint32_t tpc = 1u << lg;
     const uint32_t b0 = ((r * J.S) << lg) / 8 + 4 * (tid & (tpc - 1));
@@ -829,14 +853,14 @@ __device__ __forceinline__ void fetch_issue(Fetch& F, const LaunchArgs& args, co
 // for every store issued in between.
 __device__ __forceinline__ void consume(uint32_t v) { asm volatile("" ::"v"(v)); }
 
-template <bool kTiny, uint32_t kLg>
-__device__ __forceinline__ void fetch_commit(const Fetch& F, const LaunchArgs& args, const Job& J,
+template <bool kTiny, uint32_t kLg, class Args>
+__device__ __forceinline__ void fetch_commit(const Fetch& F, const Args& args, const Job& J,
                                              uint32_t r, uint32_t tid, uint32_t* s_tile) {
 #pragma unroll
     for (uint32_t k = 0; k < kTileBatch; ++k) consume(F.raw[k]);
     const uint32_t RB = round_len(J, r);
     if (RB == 0) return;
-    const DevTensor& T = args.t[J.d];
+    const DevTensor& T = args.tensor(J.d);
     const uint32_t lg = kLg > 0 ? kLg : J.lg;
     const uint32_t tpc = 1u << lg;
     const uint32_t i = tid & (tpc - 1);
@@ -2019,7 +2043,7 @@ constexpr uint32_t kHandoffPolls = 64;
 
 // The first half's state at its end: thread 0 writes the record's words,
 // then publishes it in word 0 (release).
-__device__ __forceinline__ void give_handoff(const LaunchArgs& args, uint32_t slot, uint32_t p0,
+__device__ __forceinline__ void give_handoff(const LaunchHead& args, uint32_t slot, uint32_t p0,
                                           uint32_t ob, uint32_t lead, const uint8_t* stage) {
     uint64_t* const rec = args.handoff + static_cast<uint64_t>(slot) * kHandoffWords;
     const uint64_t tg = static_cast<uint64_t>(args.tag) << 32;
@@ -2042,7 +2066,7 @@ __device__ __forceinline__ void give_handoff(const LaunchArgs& args, uint32_t sl
 // The second half's wait (thread 0): out[0] 1 when the record was taken,
 // then p0, the symbols placed, the carried symbols (< kGroup), their bytes.
 // A record whose values cannot come from its chunk is not taken.
-__device__ __forceinline__ void take_handoff(const LaunchArgs& args, uint32_t slot, uint32_t group,
+__device__ __forceinline__ void take_handoff(const LaunchHead& args, uint32_t slot, uint32_t group,
                                           uint32_t lim, uint32_t* out) {
     uint64_t* const rec = args.handoff + static_cast<uint64_t>(slot) * kHandoffWords;
     const uint64_t tg = static_cast<uint64_t>(args.tag) << 32;
@@ -2082,8 +2106,8 @@ __device__ __forceinline__ void take_handoff(const LaunchArgs& args, uint32_t sl
 // kLg > 0 fixes the threads per chunk at 1 << kLg for the whole launch, so
 // that sub-group geometry and the per-thread offsets derived from it are
 // compile-time constants.
-template <int kMode, int kGroup, bool kTiny, uint32_t kLg>
-__global__ __launch_bounds__(kThreads, kWavesPerSimd) void decode_kernel(const LaunchArgs args) {
+template <int kMode, int kGroup, bool kTiny, uint32_t kLg, int kN>
+__global__ __launch_bounds__(kThreads, kWavesPerSimd) void decode_kernel(const LaunchArgsN<kN> args) {
     __shared__ Lds lds;
     uint32_t* const s_wsyms = lds.wsyms;
     uint8_t* const s_wmeta = lds.wmeta;
@@ -2131,12 +2155,12 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void decode_kernel(const L
     Job cur = make_job<kMode, kLg>(args, blockIdx.x, tid);
     Fetch F;
     fetch_issue<kMode, kTiny, kLg>(F, args, cur, cur.r0, tid);
-    loaded = uniform(args.t[uniform(static_cast<uint32_t>(cur.d))].table);
+    loaded = uniform(args.tensor(uniform(static_cast<uint32_t>(cur.d))).table);
     load_table(loaded, tid, s_wsyms, s_wmeta, s_len, s_esc);
     fetch_commit<kTiny, kLg>(F, args, cur, cur.r0, tid, s_tile);
 
     for (int64_t item = blockIdx.x; item < args.total_items; item += gridDim.x) {
-        const DevTensor& T = args.t[uniform(static_cast<uint32_t>(cur.d))];
+        const DevTensor& T = args.tensor(uniform(static_cast<uint32_t>(cur.d)));
         const uint8_t* const table = uniform(T.table);
         const uint32_t lg = kLg > 0 ? kLg : uniform(cur.lg);
         const uint32_t tpc = 1u << lg;
@@ -2995,8 +3019,8 @@ __device__ __forceinline__ void run_fetch_commit(const RunFetch& F, const DevTen
 // segments number G (usable index). With stride 1 the rounds are one run
 // and a round's last partial vector group carries into the next; otherwise
 // each round stores its own partial groups element by element.
-template <int kMode, int kGroup>
-__device__ void run_piece(RunLds& lds, const Tables& tb, bool global_esc, const LaunchArgs& args,
+template <int kMode, int kGroup, class Args>
+__device__ void run_piece(RunLds& lds, const Tables& tb, bool global_esc, const Args& args,
                           const DevTensor& T, uint32_t m0, uint32_t n_rounds, uint32_t stride,
                           uint32_t G, const uint8_t* table) {
     const uint32_t s_lo = m0 * kThreads;
@@ -3153,7 +3177,7 @@ __device__ void run_piece(RunLds& lds, const Tables& tb, bool global_esc, const 
 // el_from: elements below it are left alone (the fused GEMV must not add a
 // product twice).
 template <int kMode>
-__device__ void run_fallback(const Tables& tb, const LaunchArgs& args, const DevTensor& T,
+__device__ void run_fallback(const Tables& tb, const LaunchHead& args, const DevTensor& T,
                              int64_t c_lo, int64_t c_hi, int64_t el_from = 0) {
     for (int64_t c = c_lo + threadIdx.x; c < c_hi; c += kThreads) {
         int64_t off, nb;
@@ -3183,8 +3207,8 @@ __device__ void run_fallback(const Tables& tb, const LaunchArgs& args, const Dev
     }
 }
 
-template <int kMode, int kGroup>
-__global__ __launch_bounds__(kThreads, kWavesPerSimd) void run_kernel(const LaunchArgs args) {
+template <int kMode, int kGroup, int kN>
+__global__ __launch_bounds__(kThreads, kWavesPerSimd) void run_kernel(const LaunchArgsN<kN> args) {
     __shared__ RunLds lds;
     const uint32_t tid = threadIdx.x;
     Tables tb;
@@ -3200,17 +3224,17 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void run_kernel(const Laun
     // and b + 256 share a CU, so no CU takes two extra rounds while another
     // takes none; an even split of segments instead gives every workgroup a
     // last, mostly empty round).
-    if (tid < static_cast<uint32_t>(args.n_tensors)) lds.segs[tid] = run_segments(args.t[tid]);
+    if (tid < static_cast<uint32_t>(args.count())) lds.segs[tid] = run_segments(args.tensor(tid));
     __syncthreads();
     uint64_t units = 0;
-    for (int d = 0; d < args.n_tensors; ++d)
+    for (int d = 0; d < args.count(); ++d)
         units += (static_cast<uint64_t>(lds.segs[d]) + kThreads - 1) / kThreads;
     const uint64_t per = units / gridDim.x, extra = units % gridDim.x;
     const uint64_t lo = blockIdx.x * per + (blockIdx.x < extra ? blockIdx.x : extra);
     const uint64_t hi = lo + per + (blockIdx.x < extra ? 1 : 0);
     uint64_t at = 0;  // rounds of the tensors before d
-    for (int d = 0; d < args.n_tensors; ++d) {
-        const DevTensor& T = args.t[d];
+    for (int d = 0; d < args.count(); ++d) {
+        const DevTensor& T = args.tensor(d);
         const uint32_t G = uniform(lds.segs[d]);
         const uint64_t U = (static_cast<uint64_t>(G) + kThreads - 1) / kThreads;
         const uint64_t ua = lo > at ? lo : at;
@@ -3487,8 +3511,8 @@ __device__ __forceinline__ void spec_tile_commit(const uint32_t (&raw)[kTileBatc
 }
 
 // Chunks [ca, cb) of tensor T (all of them below n_jobs).
-template <int kMode, int kGroup>
-__device__ void spec_piece(SpecLds& lds, const Tables& tb, bool global_esc, const LaunchArgs& args,
+template <int kMode, int kGroup, class Args>
+__device__ void spec_piece(SpecLds& lds, const Tables& tb, bool global_esc, const Args& args,
                            const DevTensor& T, uint32_t ca, uint32_t cb, const uint8_t* table,
                            uint32_t pre_c0 = 0xFFFFFFFFu) {
     const uint32_t tid = threadIdx.x;
@@ -3874,8 +3898,8 @@ __device__ uint32_t spec_split(const DevTensor& T, uint32_t ca, uint32_t cb, Spe
 // set) workgroups b and b + grid / 2 are taken to share a CU and split one
 // CU's share; a launch of one tensor there shares out chunks instead
 // (n_jobs b / (grid / 2) on), split by spec_split.
-template <int kMode, int kGroup>
-__global__ __launch_bounds__(kThreads, kWavesPerSimd) void spec_kernel(const LaunchArgs args) {
+template <int kMode, int kGroup, int kN>
+__global__ __launch_bounds__(kThreads, kWavesPerSimd) void spec_kernel(const LaunchArgsN<kN> args) {
     __shared__ SpecLds lds;
     Tables tb;
     tb.syms = lds.wsyms;
@@ -3887,7 +3911,7 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void spec_kernel(const Lau
     const uint32_t s = blockIdx.x % P, h = blockIdx.x / P;
     // (One call of spec_piece below: a second copy of it made the batch-4
     // GEMV's registers spill to scratch memory, 4x slower.)
-    const bool by_chunks = P != G && args.n_tensors == 1;
+    const bool by_chunks = P != G && args.count() == 1;
     uint32_t pre_c0 = 0xFFFFFFFFu;
     uint32_t ca_w = 0, cb_w = 0;  // by_chunks: this workgroup's chunks
     int64_t lo = 0, hi = 0;       // otherwise: its share of the elements
@@ -3907,8 +3931,8 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void spec_kernel(const Lau
     }
     const uint8_t* loaded = pre_c0 != 0xFFFFFFFFu ? uniform(args.t[0].table) : nullptr;
     int64_t O = 0;  // first element of tensor d in the sequence
-    for (int d = 0; d < args.n_tensors; ++d) {
-        const DevTensor& T = args.t[d];
+    for (int d = 0; d < args.count(); ++d) {
+        const DevTensor& T = args.tensor(d);
         const int64_t cs = T.chunk_size;
         int64_t ca = ca_w, cb = cb_w;
         if (!by_chunks) {
@@ -4048,6 +4072,27 @@ int plan_split(LaunchArgs& a, int64_t n, int64_t slots) {
     return AIMG_OK;
 }
 
+// f with the batch's arguments: of one tensor when it holds one (the fused
+// products' launches always do). Not for the GEMV of 2 to 4 rows of x, whose
+// registers spill with the tensor known (5120x17408 at 1024-symbol chunks
+// 96.0 -> 97.3 us).
+template <int kMode, typename F>
+void by_count(const Batch& B, F&& f) {
+    if constexpr (kMode == kModeGemv) {
+        f(B.args);
+        return;
+    } else if constexpr (kMode == kModeU8 || kMode == kModeBf16) {
+        if (B.m != 1) {
+            f(B.args);
+            return;
+        }
+    }
+    LaunchArgsN<1> one{};
+    static_cast<LaunchHead&>(one) = B.args;
+    one.t[0] = B.args.t[0];
+    f(one);
+}
+
 template <int kMode>
 int launch_batch(Batch& B, hipStream_t s, bool tiny) {
     B.args.n_tensors = B.m;
@@ -4073,21 +4118,28 @@ int launch_batch(Batch& B, hipStream_t s, bool tiny) {
     if constexpr (kMode == kModeIndex) {
         // No output: one kernel per sub-group geometry.
         if (tiny)
-            hipLaunchKernelGGL((decode_kernel<kMode, 1, true, 0>), gdim, bdim, 0, s, B.args);
+            hipLaunchKernelGGL((decode_kernel<kMode, 1, true, 0, AIMG_MAX_TENSORS>), gdim, bdim, 0, s, B.args);
         else if (B.full)
-            hipLaunchKernelGGL((decode_kernel<kMode, 1, false, kLgThreads>), gdim, bdim, 0, s, B.args);
+            hipLaunchKernelGGL((decode_kernel<kMode, 1, false, kLgThreads, AIMG_MAX_TENSORS>), gdim, bdim, 0, s,
+                               B.args);
         else
-            hipLaunchKernelGGL((decode_kernel<kMode, 1, false, 0>), gdim, bdim, 0, s, B.args);
+            hipLaunchKernelGGL((decode_kernel<kMode, 1, false, 0, AIMG_MAX_TENSORS>), gdim, bdim, 0, s, B.args);
+    } else if (tiny) {
+        hipLaunchKernelGGL((decode_kernel<kMode, 1, true, 0, AIMG_MAX_TENSORS>), gdim, bdim, 0, s, B.args);
     } else {
-    if (tiny) {
-        hipLaunchKernelGGL((decode_kernel<kMode, 1, true, 0>), gdim, bdim, 0, s, B.args);
-    } else if (B.vec && B.full) {
-        hipLaunchKernelGGL((decode_kernel<kMode, kVecGroup, false, kLgThreads>), gdim, bdim, 0, s, B.args);
-    } else if (B.vec) {
-        hipLaunchKernelGGL((decode_kernel<kMode, kVecGroup, false, 0>), gdim, bdim, 0, s, B.args);
-    } else {
-        hipLaunchKernelGGL((decode_kernel<kMode, 1, false, 0>), gdim, bdim, 0, s, B.args);
-    }
+        // (Whole-workgroup chunks keep the form for many tensors: with the
+        // tensor known their registers spill, 0.4% to 1.4% slower on the
+        // 5120x17408 layer.)
+        if (B.vec && B.full)
+            hipLaunchKernelGGL((decode_kernel<kMode, kVecGroup, false, kLgThreads, AIMG_MAX_TENSORS>), gdim, bdim,
+                               0, s, B.args);
+        else if (!B.vec)
+            hipLaunchKernelGGL((decode_kernel<kMode, 1, false, 0, AIMG_MAX_TENSORS>), gdim, bdim, 0, s, B.args);
+        else
+            by_count<kMode>(B, [&](const auto& args) {
+                constexpr int kN = sizeof(args) == sizeof(LaunchArgs) ? AIMG_MAX_TENSORS : 1;
+                hipLaunchKernelGGL((decode_kernel<kMode, kVecGroup, false, 0, kN>), gdim, bdim, 0, s, args);
+            });
     }
     const hipError_t err = hipGetLastError();
     if (err != hipSuccess)
@@ -4130,7 +4182,10 @@ int launch_run(Batch& B, hipStream_t s) {
     const int64_t want = bits / (static_cast<int64_t>(kThreads) * kMaxSegBits) + 1;
     const dim3 gdim(static_cast<uint32_t>(want < slots ? want : slots)), bdim(kThreads);
     constexpr int kVecGroup = kMode == kModeU8 ? 16 : 8;
-    hipLaunchKernelGGL((run_kernel<kMode, kVecGroup>), gdim, bdim, 0, s, B.args);
+    by_count<kMode>(B, [&](const auto& args) {
+        constexpr int kN = sizeof(args) == sizeof(LaunchArgs) ? AIMG_MAX_TENSORS : 1;
+        hipLaunchKernelGGL((run_kernel<kMode, kVecGroup, kN>), gdim, bdim, 0, s, args);
+    });
     const hipError_t err = hipGetLastError();
     if (err != hipSuccess)
         return fail(AIMG_ERR_HIP, std::string("kernel launch failed: ") + hipGetErrorString(err));
@@ -4155,8 +4210,11 @@ int launch_spec(Batch& B, hipStream_t s) {
     // A full grid: workgroups b and b + grid / 2 share a CU and split its share.
     B.args.strided = grid == slots ? 1 : 0;
     constexpr int kVecGroup = kMode == kModeU8 ? 16 : 8;
-    hipLaunchKernelGGL((spec_kernel<kMode, kVecGroup>), dim3(static_cast<uint32_t>(grid)), dim3(kThreads), 0,
-                       s, B.args);
+    by_count<kMode>(B, [&](const auto& args) {
+        constexpr int kN = sizeof(args) == sizeof(LaunchArgs) ? AIMG_MAX_TENSORS : 1;
+        hipLaunchKernelGGL((spec_kernel<kMode, kVecGroup, kN>), dim3(static_cast<uint32_t>(grid)),
+                           dim3(kThreads), 0, s, args);
+    });
     const hipError_t err = hipGetLastError();
     if (err != hipSuccess)
         return fail(AIMG_ERR_HIP, std::string("kernel launch failed: ") + hipGetErrorString(err));
