@@ -143,8 +143,12 @@ enum Mode : int {
     kModeIndex = 4, // the segment index: each segment's first boundary and codewords
     kModeGemm = 5,      // Y += X W^T for up to 16 rows of X, W decoded on the fly (MFMA)
     kModeGemmRows = 6,  // kModeGemm for rows of more than kGemmPieceMaxCols columns
+    kModeGemvShort = 8, // kModeGemv (batch 1 too) for rows of fewer than kGemvShortCols columns
     kModeGemmTile = 7,  // kModeGemm through a ring of exponents in a workspace, 16 whole rows at a time
 };
+constexpr bool is_gemv(int mode) {
+    return mode == kModeGemv || mode == kModeGemv1 || mode == kModeGemvShort;
+}
 constexpr bool is_gemm(int mode) {
     return mode == kModeGemm || mode == kModeGemmRows || mode == kModeGemmTile;
 }
@@ -157,6 +161,10 @@ constexpr bool needs_sm(int mode) { return mode != kModeU8 && mode != kModeIndex
 // Job::ib of a chunk decoded without the index.
 constexpr uint32_t kNoIndex = 0xFFFFFFFFu;
 constexpr int kGemvMaxBatch = 4;
+// Rows of fewer columns (a wave's 512 elements at one store step) take a mode
+// of their own: their code in the other two made registers spill (5120x17408
+// with 4 rows of x 87.3 -> 91.3 us).
+constexpr int64_t kGemvShortCols = 512;
 // Rows of x (tokens) of the fused decode -> GEMM: one MFMA tile's 16.
 constexpr int kGemmMaxRows = 16;
 // Steps ahead of use that x is requested with up to kGemvMaxBatch x vectors
@@ -930,6 +938,22 @@ __device__ __forceinline__ uint32_t wave_scan_incl_f32(uint32_t v) {
 }
 
 // v of the lane below (0 in lane 0; every lane active).
+// Inclusive fp32 scan over the wave that starts anew at each row: pos lanes
+// below this one belong to its row (every lane active).
+__device__ __forceinline__ float wave_rows_scan_f32(float v, uint32_t pos, uint32_t lane) {
+    auto step = [&](uint32_t below, bool in) {
+        if (in) v += __uint_as_float(below);
+    };
+    step(dpp<0x111>(__float_as_uint(v)), pos >= 1 && (lane & 15u) >= 1);
+    step(dpp<0x112>(__float_as_uint(v)), pos >= 2 && (lane & 15u) >= 2);
+    step(dpp<0x114>(__float_as_uint(v)), pos >= 4 && (lane & 15u) >= 4);
+    step(dpp<0x118>(__float_as_uint(v)), pos >= 8 && (lane & 15u) >= 8);
+    // Lane 15 of the 16 below, then lane 31, where the row reaches that far.
+    step(dpp<0x142, 0xA>(__float_as_uint(v)), (lane & 16u) != 0 && pos > (lane & 15u));
+    step(dpp<0x143, 0xC>(__float_as_uint(v)), lane >= 32 && pos > lane - 32);
+    return v;
+}
+
 __device__ __forceinline__ uint32_t lane_below(uint32_t v) { return dpp<0x138>(v); }
 
 __device__ __forceinline__ uint32_t block_scan_excl(uint32_t v, uint32_t* s_wsum) {
@@ -976,7 +1000,7 @@ __device__ __forceinline__ void store_one(const DevTensor& T, const GemvArgs& G,
         static_cast<uint8_t*>(T.out)[el] = static_cast<uint8_t>(e);
     } else if (kMode == kModeBf16) {
         static_cast<uint16_t*>(T.out)[el] = bf16_one(T.sm[el], e);
-    } else if (kMode == kModeGemv || kMode == kModeGemv1 || is_gemm(kMode)) {
+    } else if (is_gemv(kMode) || is_gemm(kMode)) {
         const float w = bf16_to_f32(bf16_one(T.sm[el], e));
         const uint32_t row = static_cast<uint32_t>(el / G.cols);
         const uint32_t col = static_cast<uint32_t>(el - static_cast<int64_t>(row) * G.cols);
@@ -1110,7 +1134,7 @@ __device__ __forceinline__ void step_rc(uint32_t& row, uint32_t& col, const Gemv
 // added to y with one atomic per x vector when the row changes. A step that
 // crosses a row boundary (about 512 / cols of them) flushes the lanes of the
 // first row and starts the next row's sums with the others. Only rows
-// shorter than 512 elements take per-lane atomics. Dead lanes' products are
+// shorter than 512 elements are summed in the wave, one atomic a row. Dead lanes' products are
 // dropped (not multiplied by zero), so an infinite x cannot make a NaN. x is
 // requested kXAhead steps ahead of use for every x vector, and every
 // vector's loads and products are unconditional (see gemv_load_x); G's x and
@@ -1120,6 +1144,8 @@ __device__ __forceinline__ void gemv_round_whole(const uint2 (&sm)[kStoreBatch],
                                                  int nb, const uint8_t* stage, uint32_t a0,
                                                  uint32_t nfull, uint32_t i, uint32_t v_lo) {
     static_assert(kThreads * kGroup == 4096, "step_rows / step_cols are for 4096 elements");
+    static_assert(kGemvShortCols == 64 * kGroup, "kGemvShortCols");
+    constexpr bool kShort = kMode == kModeGemvShort;
     constexpr uint32_t kXAhead = kB == 1 ? 3 : kGemvXAhead;
     constexpr uint32_t kSpan = 64 * kGroup;  // elements a wave holds at one step
     const uint32_t cols = G.cols;
@@ -1164,7 +1190,8 @@ __device__ __forceinline__ void gemv_round_whole(const uint2 (&sm)[kStoreBatch],
         w.y = pa.y;
         w.z = pb.x;
         w.w = pb.y;
-        if (ec + kSpan <= cols) {
+        if constexpr (!kShort) {
+            // (Once for both branches below: a copy in each was 1% slower.)
             if (er != acc_row) {
                 if (acc_row != 0xFFFFFFFFu) {
                     gemv_flush_lanes<kB>(G, nb, acc, acc_row);
@@ -1173,22 +1200,16 @@ __device__ __forceinline__ void gemv_round_whole(const uint2 (&sm)[kStoreBatch],
                 }
                 acc_row = er;
             }
+        }
+        if (!kShort && ec + kSpan <= cols) {
 #pragma unroll
             for (int b = 0; b < kB; ++b) {
                 const float t = dot8_acc(w, xc[b], acc[b]);
                 acc[b] = live ? t : acc[b];
             }
-        } else if (cols >= kSpan) {
+        } else if constexpr (!kShort) {
             // Two rows: lanes below the boundary finish row er, the rest
             // start row er + 1.
-            if (er != acc_row) {
-                if (acc_row != 0xFFFFFFFFu) {
-                    gemv_flush_lanes<kB>(G, nb, acc, acc_row);
-#pragma unroll
-                    for (int b = 0; b < kB; ++b) acc[b] = 0.0f;
-                }
-                acc_row = er;
-            }
             const bool lo = lr == er;
             float p[kB];
 #pragma unroll
@@ -1201,12 +1222,20 @@ __device__ __forceinline__ void gemv_round_whole(const uint2 (&sm)[kStoreBatch],
 #pragma unroll
             for (int b = 0; b < kB; ++b) acc[b] = lo ? 0.0f : p[b];
             acc_row = er + 1;
-        } else if (live) {
-            // Rows shorter than a wave's 512 elements: per-lane atomics.
+        } else {
+            // Rows shorter than a wave's 512 elements: a row's lanes are
+            // summed in the wave, and its last lane adds the sum (one atomic a
+            // lane instead took 271 us for 30000x256 with 4 rows of x, and
+            // 1429 for 10000x300 at 8192-symbol chunks: lanes of a row, and
+            // waves of a round, wait for each other at one address).
+            const uint32_t pos = lc / kGroup < lane ? lc / kGroup : lane;
+            const bool end = lane == 63 || lc + kGroup >= cols;
 #pragma unroll
             for (int b = 0; b < kB; ++b) {
                 if (b >= nb) break;
-                atomicAdd(G.y + static_cast<int64_t>(b) * G.rows + lr, dot8_acc(w, xc[b], 0.0f));
+                const float t = dot8_acc(w, xc[b], 0.0f);
+                const float sum = wave_rows_scan_f32(live ? t : 0.0f, pos, lane);
+                if (end && sum != 0.0f) atomicAdd(G.y + static_cast<int64_t>(b) * G.rows + lr, sum);
             }
         }
     }
@@ -1889,7 +1918,7 @@ __device__ __forceinline__ void store_round(const SmBatch<kMode>& B, const DevTe
         }
         return;
     }
-    if constexpr (kWhole && (kMode == kModeGemv || kMode == kModeGemv1)) {
+    if constexpr (kWhole && is_gemv(kMode)) {
         constexpr int kB = kMode == kModeGemv1 ? 1 : kGemvMaxBatch;
         gemv_round_whole<kMode, kGroup, kB>(sm, G, kMode == kModeGemv1 ? 1 : G.batch, stage,
                                             static_cast<uint32_t>(a0), nfull, i, v_lo);
@@ -3118,7 +3147,7 @@ __device__ void run_piece(RunLds& lds, const Tables& tb, bool global_esc, const 
         const uint32_t rem0 = avail - nfull * kGroup;
         // (The fused GEMV's rounds are never strided; compiling the path for
         // it spills its registers to scratch.)
-        if (kMode != kModeGemv && kMode != kModeGemv1 && stride != 1) {
+        if (!is_gemv(kMode) && stride != 1) {
             // Rounds of other workgroups follow: the partial group goes out
             // element by element (the elements before `skip` of a round's
             // first group are the previous round's).
@@ -3257,7 +3286,7 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void run_kernel(const Laun
         tb.min_len = hdr->min_len >= 1 ? hdr->min_len : 1u;
         tb.gesc = (const __attribute__((address_space(1))) uint16_t*)(table + kEscOffset);
         const bool global_esc = hdr->n_esc_blocks > static_cast<uint32_t>(kLdsEscBlocks);
-        if (kMode != kModeGemv && kMode != kModeGemv1 && G != 0 && args.strided) {
+        if (!is_gemv(kMode) && G != 0 && args.strided) {
             // Rounds u = blockIdx.x + k * grid of the launch's round sequence.
             const uint64_t first = at + (blockIdx.x + gridDim.x - at % gridDim.x) % gridDim.x;
             if (first < at + U) {
@@ -4173,7 +4202,7 @@ int launch_run(Batch& B, hipStream_t s) {
     // selects contiguous ranges for the decodes too.
     const char* st = std::getenv("AIMG_RUN_STRIDED");
     B.args.strided =
-        (kMode == kModeGemv || kMode == kModeGemv1) || (st != nullptr && st[0] == '0') ? 0 : 1;
+        is_gemv(kMode) || (st != nullptr && st[0] == '0') ? 0 : 1;
     int64_t bits = 0;
     for (int d = 0; d < B.m; ++d) bits += 8 * B.args.t[d].packed_nbytes;
     // A workgroup per round (of 168-bit segments) up to a full grid: each
@@ -4312,14 +4341,17 @@ int check_tensor(const aimg_tensor& t) {
 
 // Whether the ring serves an n_x-row GEMM faster than the modes without it
 // (microseconds without, with; 1024-symbol chunks unless said). Rows of more
-// than kGemmPieceMaxCols columns: always (4x20480, 16 rows of x: 37, 18;
-// 3000x20480: 249, 77). Shorter ones: X is read once a piece of 2048 groups
+// than kGemmPieceMaxCols columns: but for a handful of rows (4x20480, 16 rows
+// of x: 37, 18; 3000x20480: 249, 77; 20x9000, 5 rows: 26, 22; 8x12000 at
+// 16384 symbols: 23, 26). Shorter ones: X is read once a piece of 2048 groups
 // without the ring, which costs more with more rows of x and more columns.
 // 16 rows: 30000x1000 43, 48; 30000x1400 61, 59; 8000x2048 36, 32; 800x5120
 // 26, 23. 5 rows: 8000x2048 31, 32; 30000x2048 71, 70; 800x5120 21, 23;
 // 2000x4096 26, 25; 4096x4096 at 65536 symbols 38, 32. n_x 0: not asked.
-bool ring_pays(int64_t n_symbols, int64_t cols, int n_x) {
-    if (n_x == 0 || cols > kGemmPieceMaxCols) return true;
+bool ring_pays(int64_t n_symbols, int64_t rows, int64_t cols, int n_x) {
+    if (n_x == 0) return true;
+    if (rows < 12 && n_x <= 8) return false;
+    if (cols > kGemmPieceMaxCols) return true;
     if (n_x > 8) return cols >= 2048;
     return cols >= 4096 && n_symbols >= (int64_t{1} << 23);
 }
@@ -4344,8 +4376,9 @@ RingPlan plan_ring(int64_t n_symbols, int64_t cols, int64_t chunk_size) {
     const int64_t chunks = (n_symbols + chunk_size - 1) / chunk_size;
     P.grid = chunks < slots ? chunks : slots;
     if (P.grid < 1) return P;
-    // (launch_spec: a workgroup's chunks are at most a CU's share, rounded up.)
-    const int64_t cus = P.grid == slots && slots % 2 == 0 ? slots / 2 : P.grid;
+    // (launch_spec, whichever grid it takes: a workgroup's chunks are at most
+    // one of slots / 2 shares of them, rounded up.)
+    const int64_t cus = chunks < slots / 2 || slots < 2 ? chunks : slots / 2;
     const int64_t share = (chunks / cus + 2) * chunk_size;
     const int64_t need = kTileRows + (kRingRound + cols - 1) / cols;
     const int64_t all = (share < n_symbols ? share : n_symbols) / cols + 2;
@@ -4573,6 +4606,7 @@ extern "C" int aimg_decode_gemv_bf16(const aimg_tensor* t, int64_t rows, int64_t
     // The 8-weight groups take 16-byte x loads: they must lie inside one row
     // (cols % 8 == 0) and x must be 16-byte aligned.
     const bool vec_ok = cols % 8 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0;
+    if (cols < aimg::kGemvShortCols) return aimg::launch<aimg::kModeGemvShort>(t, 1, g, vec_ok, stream);
     if (batch == 1) return aimg::launch<aimg::kModeGemv1>(t, 1, g, vec_ok, stream);
     return aimg::launch<aimg::kModeGemv>(t, 1, g, vec_ok, stream);
 }
@@ -4618,7 +4652,7 @@ extern "C" int aimg_gemm_workspace_nbytes(const aimg_tensor* t, int64_t rows, in
     if (n_x < 0 || n_x > aimg::kGemmMaxRows)
         return fail(AIMG_ERR_INVALID_ARGUMENT, "n_x must be in 0.." + std::to_string(aimg::kGemmMaxRows));
     *nbytes = 0;
-    if (cols % 8 != 0 || t->chunk_size < 8 || !aimg::ring_pays(t->n_symbols, cols, n_x)) return AIMG_OK;
+    if (cols % 8 != 0 || t->chunk_size < 8 || !aimg::ring_pays(t->n_symbols, rows, cols, n_x)) return AIMG_OK;
     *nbytes = aimg::plan_ring(t->n_symbols, cols, t->chunk_size).nbytes;
     return AIMG_OK;
 }

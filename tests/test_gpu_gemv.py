@@ -88,3 +88,22 @@ def test_accumulates_into_given_y_and_rejects_bad_shapes():
         decode_gemv(t, x, 8, 64)
     with pytest.raises(ValueError, match="2-D"):
         decompress_matvec_gpu(compress_layer(W.reshape(-1)), x[0])
+
+
+@pytest.mark.parametrize("batch", [1, 3])
+@pytest.mark.parametrize("shape,chunk", [((900, 8), 1024), ((2000, 136), 128), ((700, 504), 65536),
+                                         ((5000, 256), 2048), ((300, 512), 1000)])
+def test_short_rows(shape, chunk, batch):
+    """Rows of fewer than a wave step's 512 columns, whose lanes are summed in
+    the wave (and 512, which are not), against 64 bits: at most one rounding a
+    term in any order, |error| <= cols * 2^-24 * sum |w x|."""
+    W = workloads.bf16_normal(shape, 7 + batch, 0.02, outlier_frac=1e-3)
+    layer = compress_layer(W, chunk_size=chunk)
+    g = np.random.default_rng(batch)
+    x = torch.from_numpy(g.standard_normal((batch, shape[1]), dtype=np.float32)).to(torch.bfloat16)
+    t = DeviceTensor.from_encoded(layer.encoded, layer.sign_mantissa, "cuda")
+    for _ in range(2):
+        y = decode_gemv(t, x.cuda(), *shape).cpu().double()
+        bound = shape[1] * 2.0 ** -24 * (x.double().abs() @ W.double().abs().t()) + 1e-30
+        assert bool(((y - x.double() @ W.double().t()).abs() <= bound).all())
+        t.build_index()  # the second pass with the segment index (chunks it serves)

@@ -606,3 +606,11 @@ def test_fused_gemm(emu, rows, cols, chunk, n_x):
 def test_fused_gemm_ring(emu, rows, cols, chunk, n_x, cus):
     _gemv(emu, "ring_%d_%d_%d_%d" % (rows, cols, chunk, n_x), rows, cols, chunk, n_x, 40 + n_x,
           cus=cus, mode="gemm-ring")
+
+
+# GEMV rows shorter than a wave step's 512 elements (a row's lanes summed in
+# the wave): rows of one group, of lane counts that cross 16 and 32 lanes.
+
+@pytest.mark.parametrize("rows,cols,batch", [(900, 8, 2), (40, 504, 1), (120, 136, 4)])
+def test_gemv_short_rows(emu, rows, cols, batch):
+    _gemv(emu, "gshort_%d" % cols, rows, cols, 1024, batch, 31, cus=1)
