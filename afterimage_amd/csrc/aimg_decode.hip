@@ -3319,7 +3319,7 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void run_kernel(const Laun
 
 // ---------------------------------------------------------------------------
 // Speculative segment runs: decode without an index of tensors whose chunks
-// hold kRunMinChunk symbols or more (vector path).
+// hold kSpecMinChunk symbols or more (vector path).
 //
 // A workgroup takes a contiguous range of the launch's chunks and walks it in
 // rounds of 512 segments that run across chunk boundaries: segment k of a
@@ -4221,9 +4221,22 @@ int launch_run(Batch& B, hipStream_t s) {
     return AIMG_OK;
 }
 
+// Workgroups of a speculative launch: one per chunk up to two per CU, and one
+// per CU where that leaves none more than about a round of segments: it then
+// decodes as long alone as with another beside it, and half of the start-ups
+// and table loads fall away (1024x3072 at 4096-symbol chunks 12.1 -> 11.6 us,
+// 400x1000 at 1024 12.8 -> 11.0; one workgroup per round, 96 of them, 18.4).
+int64_t spec_grid(const Batch& B, int64_t chunks, int64_t slots) {
+    int64_t bits = 0;
+    for (int d = 0; d < B.m; ++d) bits += 8 * B.args.t[d].packed_nbytes;
+    const bool one_round = bits / (static_cast<int64_t>(kThreads) * kMaxSegBits) + 1 < slots / 2;
+    const int64_t most = one_round && slots > 1 ? slots / 2 : slots;
+    return chunks < most ? chunks : most;
+}
+
 // The speculative segment-run kernel over the batch's tensors: each workgroup
 // takes the chunks whose first element lies in its share of the tensors'
-// elements (a grid of one workgroup per chunk up to two per CU).
+// elements.
 template <int kMode>
 int launch_spec(Batch& B, hipStream_t s) {
     if (B.m == 0) return AIMG_OK;
@@ -4235,7 +4248,7 @@ int launch_spec(Batch& B, hipStream_t s) {
     }
     B.args.total_items = elements;
     const int64_t slots = static_cast<int64_t>(cu_count()) * kBlocksPerCu;
-    const int64_t grid = chunks < slots ? chunks : slots;
+    const int64_t grid = spec_grid(B, chunks, slots);
     // A full grid: workgroups b and b + grid / 2 share a CU and split its share.
     B.args.strided = grid == slots ? 1 : 0;
     constexpr int kVecGroup = kMode == kModeU8 ? 16 : 8;
@@ -4252,10 +4265,19 @@ int launch_spec(Batch& B, hipStream_t s) {
 
 // Tensors with a segment index (chunks of kRunMinChunk symbols or more, the
 // vector path's alignment) go to `run`, the segment-run kernel, when `run`
-// is given; tensors without one that meet the same conditions go to `spec`,
-// the speculative segment-run kernel, when `spec` is given; the others decode
-// chunk by chunk.
+// is given; tensors without one that meet the same alignment, with chunks of
+// kSpecMinChunk symbols or more, go to `spec`, the speculative segment-run
+// kernel, when `spec` is given; the others decode chunk by chunk.
 constexpr uint32_t kSpecMaxTpc = 128;
+// Smallest chunks the speculative runs take. A round's table holds 64 chunks,
+// so chunks of fewer than about 512 symbols leave threads without a segment,
+// but a chunk of its own (16 threads or more a chunk, most of them idle in
+// its last round) costs more still. Chunk by chunk against speculative runs:
+// 17408x5120 at 512 symbols bf16 120 -> 71 us, GEMV of 1 and 4 rows of x 153
+// -> 79 and 213 -> 100, of 4 rows at 1000 symbols 173 -> 96; 3001x4099
+// exponent bytes at 512, 256 and 128 symbols 20.5 -> 16.8, 32.4 -> 22.1 and
+// 57 -> 33.
+constexpr int32_t kSpecMinChunk = 128;
 
 template <int kMode>
 int add_tensor(const aimg_tensor& t, int i, Batch& normal, Batch& tiny, Batch* run = nullptr,
@@ -4296,7 +4318,8 @@ int add_tensor(const aimg_tensor& t, int i, Batch& normal, Batch& tiny, Batch* r
     // speculative runs against chunk by chunk: 64Ki-, 32Ki- and 16Ki-symbol
     // chunks 6%, 13% and 5% slower; 8Ki and 4Ki 3% and 11% faster).
     const bool spec_size = spec_all || threads_per_chunk(t.chunk_size) <= kSpecMaxTpc;
-    const bool to_spec = !to_run && spec != nullptr && t.chunk_size >= kRunMinChunk &&
+    const bool to_spec = !to_run && spec != nullptr &&
+                         t.chunk_size >= (is_gemm(kMode) ? kRunMinChunk : kSpecMinChunk) &&
                          t.chunk_size <= (1 << 24) && spec_size &&
                          t.packed_nbytes >= 4 && t.packed_nbytes < (int64_t{1} << 32) - (int64_t{1} << 20) &&
                          vec_layout;

@@ -188,3 +188,24 @@ def test_segment_guesses_all_wrong():
     rng = np.random.default_rng(8)
     _check(rng.integers(0, 8, 20000), chunk_size=4096)
     _check(rng.integers(0, 8, 70000), chunk_size=65536)
+
+
+@pytest.mark.parametrize("chunk", [120, 128, 136, 256, 520, 1000, 1016])
+@pytest.mark.parametrize("n", [1, 5000, 200003, 12000000])
+def test_chunks_below_1024_symbols(chunk, n, monkeypatch):
+    """bf16 and exponent bytes of chunks on both sides of the smallest that
+    take the speculative runs, at grids of a workgroup a chunk, one and two a
+    CU, against the original and against the decode chunk by chunk."""
+    from afterimage_amd import workloads
+    from afterimage_amd.runtime.compressed_store import compress_layer
+    from afterimage_amd.runtime.device import DeviceTensor, decode_bf16, decode_u8
+    W = workloads.bf16_normal((n,), chunk + n % 7, 0.02, outlier_frac=1e-3)
+    layer = compress_layer(W, chunk_size=chunk)
+    t = DeviceTensor.from_encoded(layer.encoded, layer.sign_mantissa, "cuda")
+    want = W.view(torch.int16)
+    got = decode_bf16([t])[0].cpu().view(torch.int16)
+    u8 = decode_u8([t])[0].cpu()
+    assert torch.equal(got, want)
+    assert torch.equal(u8, ((want.int() >> 7) & 0xFF).to(torch.uint8))
+    monkeypatch.setenv("AIMG_SPEC_RUNS", "0")
+    assert torch.equal(decode_bf16([t])[0].cpu().view(torch.int16), want)

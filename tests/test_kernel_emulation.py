@@ -608,6 +608,24 @@ def test_fused_gemm_ring(emu, rows, cols, chunk, n_x, cus):
           cus=cus, mode="gemm-ring")
 
 
+# Speculative runs of chunks of 128 to 1023 symbols: a round's 64-chunk table
+# ends before its 512 segments do; ragged last chunks; one-bit codes (segments
+# of 80 bits); a grid of one workgroup a CU and a full one (few and many CUs).
+
+@pytest.mark.parametrize("chunk,n,cus", [(128, 30001, 1), (136, 20000, 2), (520, 40003, 1), (1000, 50000, 40)])
+def test_spec_small_chunks_bf16(emu, chunk, n, cus):
+    W = workloads.bf16_normal((n,), chunk, 0.02, outlier_frac=1e-3)
+    _bf16(emu, "spsm_%d" % chunk, W, chunk, cus=cus)
+
+
+def test_spec_small_chunks_one_bit_codes(emu):
+    _u8(emu, "spsm_one", np.full(20000, 117), 128, cus=1)
+
+
+def test_spec_small_chunks_gemv(emu):
+    _gemv(emu, "spsm_gemv", 130, 200, 136, 3, 21, cus=1)
+
+
 # GEMV rows shorter than a wave step's 512 elements (a row's lanes summed in
 # the wave): rows of one group, of lane counts that cross 16 and 32 lanes.
 
