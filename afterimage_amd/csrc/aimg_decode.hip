@@ -4226,11 +4226,18 @@ int launch_run(Batch& B, hipStream_t s) {
 // decodes as long alone as with another beside it, and half of the start-ups
 // and table loads fall away (1024x3072 at 4096-symbol chunks 12.1 -> 11.6 us,
 // 400x1000 at 1024 12.8 -> 11.0; one workgroup per round, 96 of them, 18.4).
-int64_t spec_grid(const Batch& B, int64_t chunks, int64_t slots) {
+int64_t spec_grid(const Batch& B, int64_t chunks, int64_t slots, bool gemm) {
     int64_t bits = 0;
     for (int d = 0; d < B.m; ++d) bits += 8 * B.args.t[d].packed_nbytes;
     const bool one_round = bits / (static_cast<int64_t>(kThreads) * kMaxSegBits) + 1 < slots / 2;
-    const int64_t most = one_round && slots > 1 ? slots / 2 : slots;
+    int64_t most = one_round && slots > 1 ? slots / 2 : slots;
+    // A wave's worth of segments at least (a tiny tensor's chunks of a few
+    // segments each would load the decode table once a chunk). The fused
+    // GEMM's rings are sized for a workgroup a chunk.
+    if (!gemm) {
+        const int64_t waves = bits / (int64_t{64} * kMaxSegBits) + 1;
+        most = waves < most ? waves : most;
+    }
     return chunks < most ? chunks : most;
 }
 
@@ -4248,7 +4255,7 @@ int launch_spec(Batch& B, hipStream_t s) {
     }
     B.args.total_items = elements;
     const int64_t slots = static_cast<int64_t>(cu_count()) * kBlocksPerCu;
-    const int64_t grid = spec_grid(B, chunks, slots);
+    const int64_t grid = spec_grid(B, chunks, slots, is_gemm(kMode));
     // A full grid: workgroups b and b + grid / 2 share a CU and split its share.
     B.args.strided = grid == slots ? 1 : 0;
     constexpr int kVecGroup = kMode == kModeU8 ? 16 : 8;
