@@ -173,7 +173,9 @@ constexpr int kGemmMaxRows = 16;
 constexpr uint32_t kGemvXAhead = 1;
 
 struct GemvArgs {
-    const uint16_t* x;  // bf16 [batch][cols] (GEMM: [rows of x][cols])
+    // bf16 [batch][cols] (GEMM: [rows of x][cols]); kModeGemmTile: as
+    // pack_x_kernel leaves it, [column groups of 8][rows of x][8].
+    const uint16_t* x;
     float* y;           // fp32 [batch][rows], accumulated
     uint32_t rows;
     uint32_t cols;
@@ -192,7 +194,7 @@ struct LaunchHead {
     // Segment runs: workgroup w takes rounds w, w + grid, ... Speculative
     // runs: a full grid, whose workgroups b and b + grid / 2 split a CU's share.
     int32_t strided;
-    GemvArgs gemv;  // kModeGemv only (one tensor)
+    GemvArgs gemv;  // GEMV and GEMM modes only (one tensor)
     // Chunk by chunk, whole-workgroup chunks: the last n_split chunks (from
     // chunk item split_first on) are split in two halves of their rounds.
     // Items 0 .. n_split - 1 are their first halves, the grid's first items;
@@ -1004,9 +1006,13 @@ __device__ __forceinline__ void store_one(const DevTensor& T, const GemvArgs& G,
         const float w = bf16_to_f32(bf16_one(T.sm[el], e));
         const uint32_t row = static_cast<uint32_t>(el / G.cols);
         const uint32_t col = static_cast<uint32_t>(el - static_cast<int64_t>(row) * G.cols);
-        for (int b = 0; b < G.batch; ++b)
-            atomicAdd(G.y + static_cast<int64_t>(b) * G.rows + row,
-                      w * bf16_to_f32(G.x[static_cast<int64_t>(b) * G.cols + col]));
+        for (int b = 0; b < G.batch; ++b) {
+            // (kModeGemmTile: x is packed, a column group of every row in turn.)
+            const uint64_t at = kMode == kModeGemmTile
+                                    ? (static_cast<uint64_t>(col >> 3) * G.batch + b) * 8 + (col & 7u)
+                                    : static_cast<uint64_t>(b) * G.cols + col;
+            atomicAdd(G.y + static_cast<int64_t>(b) * G.rows + row, w * bf16_to_f32(G.x[at]));
+        }
     }
 }
 
@@ -1645,9 +1651,9 @@ __device__ __forceinline__ void ring_put(Ring& R, const uint8_t* stage, uint32_t
     if (R.at >= R.nbytes) R.at -= R.nbytes;
 }
 
-// X for ring_products, and Y's first value. packed: for each 32 columns and
-// each quarter q of them, column group q of every row of X (16 bytes a row),
-// zero past the columns; y (when zero_y) is cleared.
+// X for ring_products (and for store_one on the exact path), and Y's first
+// value. packed: for each column group (8 columns), its 16 bytes of every row
+// of X in turn, zero past the columns; the n_y first values of y are cleared.
 __global__ __launch_bounds__(256) void pack_x_kernel(const uint16_t* x, uint32_t nb, uint32_t cols,
                                                      uint32_t n_groups, uint16_t* packed, float* y,
                                                      int64_t n_y) {

@@ -13,6 +13,7 @@ from afterimage_amd import _native, workloads
 from afterimage_amd.runtime.compressed_store import (compress_layer, decompress_linear_gpu,
                                                      decompress_matvec_gpu)
 from afterimage_amd.runtime.device import GEMM_MAX_ROWS, DeviceTensor, decode_gemm
+from tests.edited_streams import LOSSLESS, edited
 
 pytestmark = pytest.mark.gpu
 
@@ -166,3 +167,16 @@ def test_ring_infinite_x():
     y = decode_gemm(t, x.cuda(), 64, 10000).cpu()
     assert bool(torch.isposinf(y[2]).all())
     assert bool(torch.isfinite(y[[0, 1, 3, 4, 5]]).all())
+
+
+@pytest.mark.parametrize("kind", LOSSLESS)
+@pytest.mark.parametrize("shape,chunk,n_x", [((600, 5120), 1024, 12), ((300, 9000), 8192, 3)])
+def test_ring_chunks_not_back_to_back(shape, chunk, n_x, kind):
+    """A workgroup that meets a chunk out of order or after a gap leaves its
+    ring for the exact path there: the same sums."""
+    W = workloads.bf16_normal(shape, 90, 0.02, outlier_frac=1e-3)
+    layer = compress_layer(W, chunk_size=chunk)
+    x = _x(n_x, shape[1], 6)
+    t = DeviceTensor.from_encoded(edited(layer.encoded, kind), layer.sign_mantissa, "cuda")
+    y = decode_gemm(t, x.cuda(), *shape).cpu().double()
+    assert bool(((y - x.double() @ W.double().t()).abs() <= _ring_bound(W, x)).all())

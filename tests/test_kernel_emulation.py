@@ -24,6 +24,7 @@ from afterimage_amd import workloads
 from afterimage_amd.runtime.compressed_store import compress_layer
 from afterimage_amd.runtime.huffman_chunked import encode_chunked
 from tests.distributions import many_escape_windows
+from tests.edited_streams import LOSSLESS, LOSSY, edited
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -606,6 +607,39 @@ def test_fused_gemm(emu, rows, cols, chunk, n_x):
 def test_fused_gemm_ring(emu, rows, cols, chunk, n_x, cus):
     _gemv(emu, "ring_%d_%d_%d_%d" % (rows, cols, chunk, n_x), rows, cols, chunk, n_x, 40 + n_x,
           cus=cus, mode="gemm-ring")
+
+
+# The same GEMMs of streams that leave the ring early for the exact path: a
+# workgroup's ring is then flushed with whatever rows it holds, and the exact
+# path adds the rest, each weight once. Chunks swapped, a gap before one, an
+# empty one (in the middle, and first of a workgroup's), a last one cut short,
+# and a re-packed stream whose chunks all miss their last byte (back to back,
+# so that rounds decode until one does not hold its symbols).
+
+def _gemm_edited(emu, name, rows, cols, chunk, n_x, kind, mode, cus):
+    import oracle
+    W = workloads.bf16_normal((rows, cols), 60, 0.02, outlier_frac=1e-3)
+    layer = compress_layer(W, chunk_size=chunk)
+    enc = edited(layer.encoded, kind)
+    sm = layer.sign_mantissa.numpy().astype(np.int32).reshape(-1)
+    e = oracle.decode_chunks(enc)[: rows * cols].astype(np.int32)
+    bits = ((sm & 0x80) << 8) | (e << 7) | (sm & 0x7F)
+    Wd = torch.from_numpy(bits.astype(np.uint16).view(np.int16)).view(torch.bfloat16).view(rows, cols)
+    if kind in LOSSLESS:
+        assert torch.equal(Wd.view(torch.int16), W.view(torch.int16))
+    x = torch.from_numpy(np.random.default_rng(61).standard_normal((n_x, cols), dtype=np.float32)).to(torch.bfloat16)
+    d = emu[1] / name
+    _write(d, enc, np.zeros(1, np.uint8), layer.sign_mantissa.numpy())
+    x.view(torch.int16).numpy().tofile(os.path.join(d, "x.bin"))
+    (x.double() @ Wd.double().t()).float().numpy().tofile(os.path.join(d, "expect_y.bin"))
+    with open(os.path.join(d, "gemv.txt"), "w") as f:
+        f.write("%d %d %d\n" % (rows, cols, n_x))
+    _run(emu, name, mode, cus=cus)
+
+
+@pytest.mark.parametrize("kind", LOSSLESS + LOSSY)
+def test_fused_gemm_ring_exact_path(emu, kind):
+    _gemm_edited(emu, "ringx_%s" % kind, 40, 5120, 4096, 6, kind, "gemm-ring", 1)
 
 
 # Speculative runs of chunks of 128 to 1023 symbols: a round's 64-chunk table
