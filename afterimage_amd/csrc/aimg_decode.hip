@@ -156,6 +156,11 @@ constexpr bool is_gemm(int mode) {
 constexpr bool keeps_tile_sums(int mode) { return mode == kModeGemm || mode == kModeGemmRows; }
 // Modes that read sign/mantissa bytes outside the round's own requests.
 constexpr bool reads_sm_late(int mode) { return mode == kModeGemmRows || mode == kModeGemmTile; }
+// Modes whose speculative rounds gather the words of chunks that are not back
+// to back. Not the GEMMs, which leave such chunks to the exact path: with the
+// gather in their rounds registers spill (151936x5120 with 8 rows of x 678 ->
+// 696 us, 5120x17408 with 16 97.5 -> 99.5).
+constexpr bool gathers(int mode) { return !is_gemm(mode); }
 // Modes that combine the exponents with sign/mantissa bytes.
 constexpr bool needs_sm(int mode) { return mode != kModeU8 && mode != kModeIndex; }
 // Job::ib of a chunk decoded without the index.
@@ -3342,6 +3347,16 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void run_kernel(const Laun
 // round's output is therefore one run of elements, compacted in LDS and
 // stored whole, as the segment runs with an index store theirs.
 //
+// A round's words are requested before its table is known, from where its
+// chunks are if they lie back to back, as encoders write them. A table whose
+// chunks do not (in another order, or padded to an alignment) makes its round
+// gather its words, chunk by chunk, once the table is there (its loads are
+// waited for; with the exact path instead, one thread a chunk, 17408x5120 took
+// 30 to 150 times as long). Microseconds back to back, padded to 16 bytes,
+// shuffled: bf16 at 512 symbols 77, 85, 94 (chunk by chunk: 120 whatever the
+// layout), at 128 184, 228, 231 (409), at 1024 72, 87, 88, GEMV of 4 rows of x
+// at 512 101, 118, 119 (213).
+//
 // The threads' slots are interleaved by lane: word j of lane l of wave w sits
 // at row j, column l of the wave's block, so the lanes of a wave write and
 // read their slots in 64 different banks whatever their positions.
@@ -3362,6 +3377,10 @@ static_assert(kSpecStageBytes >= kLeadBytes + kWaves * kSliceBytes, "a ring tile
 // fallback decodes it): segment counts come from a multiply-high that is
 // exact below it, and its bit count fits 32 bits.
 constexpr int64_t kSpecMaxChunkBytes = int64_t{1} << 26;
+// Segments of a round that gathers its words: each chunk of its table may take
+// a word more than its segments.
+constexpr uint32_t kGatherSegs = kThreads - 16;
+static_assert((kThreads - kGatherSegs) * kMaxSegBits >= 32 * (kSpecChunks + 1), "a gathered round fits the tile");
 
 struct __attribute__((aligned(16))) SpecLds {
     uint8_t wmeta[kWinEntries];
@@ -3372,10 +3391,12 @@ struct __attribute__((aligned(16))) SpecLds {
     // sets (this round's and the next one's). cseg: a chunk's first segment
     // counted from the round's first ([kSpecChunks]: the end of the table's
     // segments); coff: byte offset ([kSpecChunks]: the table's last byte + 1);
-    // cbits: bits.
+    // cbits: bits. A table whose chunks are not back to back: coff counts from
+    // the round's first byte as the words lie in the tile, src is the offset.
     int32_t cseg[2][kSpecChunks + 1];
     uint32_t coff[2][kSpecChunks + 1];
     uint32_t cbits[2][kSpecChunks];
+    uint32_t src[2][kSpecChunks];
     // Per wave, from its last lane: codewords, the wave-exclusive count of its
     // last chunk head + 1 (0: none), that lane's end, disagreement inside the
     // wave. From lane 0: its start and whether that start is known.
@@ -3434,7 +3455,9 @@ __device__ __forceinline__ void spec_tab_issue(SpecTabFetch& F, const DevTensor&
 struct SpecTab {
     uint32_t n_tab;  // chunks of the table (those below the piece's end)
     uint32_t ns;     // segments of the round (at most 512: those of the table's chunks)
-    uint32_t bad;    // 1: chunks not back to back, empty, or too large
+    uint32_t bad;    // 1: a chunk of it is empty or too large (or, without the
+                     // gather, not back to back with the one before)
+    uint32_t apart;  // 1: its chunks are not back to back (the round gathers its words)
     uint32_t off0;   // byte offset of the table's first chunk
     // The next round: its first segment is segment ns of this one, in table
     // chunk `done` (n_tab: the chunk after the table), at segment k0n of it,
@@ -3451,10 +3474,13 @@ __device__ __forceinline__ uint32_t div_ceil_seg(uint32_t a, uint32_t d, uint32_
 
 // The fetched chunks into table set `set` (written by one wave; every wave
 // computes the same result). k0: the round's first segment in chunk c0;
-// first_off: where chunk c0 must start (the previous table's view of it).
+// first_off: where chunk c0 starts if it follows the previous table's last
+// chunk (check_first: the round's words were requested from there).
 // *jj: the table chunk of the calling thread's segment (thread 64 w + lane),
 // found in registers: the chunks that start before the wave's first segment,
-// and a mask of those that start inside the wave.
+// and a mask of those that start inside the wave. kGather: the round can
+// gather its words.
+template <bool kGather>
 __device__ __forceinline__ SpecTab spec_tab_commit(const SpecTabFetch& F, const DevTensor& T,
                                                    SpecLds& lds, uint32_t set, uint32_t c0,
                                                    uint32_t cb, uint32_t k0, uint32_t first_off,
@@ -3474,9 +3500,9 @@ __device__ __forceinline__ SpecTab spec_tab_commit(const SpecTabFetch& F, const 
     const int64_t lim = T.n_symbols - static_cast<int64_t>(c) * T.chunk_size;
     const uint32_t incl = wave_scan_incl(nseg);
     const uint32_t prev_end = lane_below(offv + nbv);
-    const bool bad = valid && (huge || (nseg == 0 && lim > 0) ||
-                               (lane > 0 && offv != prev_end) ||
-                               (lane == 0 && check_first && offv != first_off));
+    const bool jump = valid && offv != (lane > 0 ? prev_end : check_first ? first_off : offv);
+    const bool bad = valid && (huge || (nseg == 0 && lim > 0) || (!kGather && jump));
+    const bool apart = kGather && __ballot(jump) != 0;
     const uint64_t vm = __ballot(valid);
     const uint32_t n_tab = static_cast<uint32_t>(__builtin_popcountll(vm));  // lanes 0 .. n_tab - 1
     const uint32_t total = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(incl), 63));
@@ -3486,7 +3512,8 @@ __device__ __forceinline__ SpecTab spec_tab_commit(const SpecTabFetch& F, const 
     const uint32_t off0 = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(offv), 0));
     const int32_t first = static_cast<int32_t>(incl - nseg) - static_cast<int32_t>(k0);
     const int32_t end = static_cast<int32_t>(total) - static_cast<int32_t>(k0);
-    const uint32_t ns = end <= 0 ? 0u : (end < static_cast<int32_t>(kThreads) ? static_cast<uint32_t>(end) : kThreads);
+    const uint32_t most = apart ? kGatherSegs : static_cast<uint32_t>(kThreads);
+    const uint32_t ns = end <= 0 ? 0u : (end < static_cast<int32_t>(most) ? static_cast<uint32_t>(end) : most);
     const uint32_t done = static_cast<uint32_t>(__builtin_popcountll(
         __ballot(valid && static_cast<int32_t>(incl) - static_cast<int32_t>(k0) <= static_cast<int32_t>(ns))));
     const uint32_t k0n = done < n_tab ? ns - static_cast<uint32_t>(__builtin_amdgcn_readlane(
@@ -3505,15 +3532,24 @@ __device__ __forceinline__ SpecTab spec_tab_commit(const SpecTabFetch& F, const 
     const uint32_t cnt = before + static_cast<uint32_t>(__builtin_popcountll(heads & upto));
     *jj = cnt > 0 ? cnt - 1 : 0u;
     if (w == 0) {
+        uint32_t at = valid ? offv : end_off;
+        if (apart) {
+            // Each chunk on a word of its own, a word more than its segments
+            // take before it: past the bytes of the one before.
+            lds.src[set][lane] = offv;
+            const uint32_t from = check_first ? first_off : off0;
+            const uint32_t f = first < 2048 ? static_cast<uint32_t>(first) : 2048u;
+            at = lane == 0 ? from : from + k0 * (S / 8) + (valid ? 4 * ((f * S + 31) / 32 + lane) : 0x0FFFFFFFu);
+        }
         lds.cseg[set][lane] = first;
-        lds.coff[set][lane] = valid ? offv : end_off;
+        lds.coff[set][lane] = at;
         lds.cbits[set][lane] = 8 * nbv;
         if (lane == 0) {
             lds.cseg[set][kSpecChunks] = static_cast<int32_t>(total) - static_cast<int32_t>(k0);
             lds.coff[set][kSpecChunks] = end_off;
         }
     }
-    return {n_tab, uniform(ns), any_bad || ns == 0 ? 1u : 0u, uniform(off0), uniform(done),
+    return {n_tab, uniform(ns), any_bad || ns == 0 ? 1u : 0u, uniform(apart ? 1u : 0u), uniform(off0), uniform(done),
             uniform(k0n), uniform(offn)};
 }
 
@@ -3545,6 +3581,41 @@ __device__ __forceinline__ void spec_tile_commit(const uint32_t (&raw)[kTileBatc
     }
 }
 
+// The words of a round whose chunks are not back to back (A0: its first byte
+// as the table counts): word j of the tile is from the last chunk whose place
+// is at or before it. Every thread calls it, past the last read of the tile;
+// a barrier follows.
+__device__ __forceinline__ void spec_tile_gather(const DevTensor& T, SpecLds& lds, uint32_t set, uint32_t A0,
+                                                 uint32_t tid) {
+    asm volatile("" : "+v"(tid));  // nothing here is kept in registers over the rounds
+    const __amdgpu_buffer_rsrc_t rs = buffer_of(T.packed, T.packed_n32);
+    const uint32_t last = last_word(T);
+    uint32_t A[kTileBatch], raw[kTileBatch];
+#pragma unroll
+    for (uint32_t k = 0; k < kTileBatch; ++k) {
+        const uint32_t at = 4 * (k * kThreads + tid);
+        uint32_t c = 0;
+#pragma unroll
+        for (uint32_t step = kSpecChunks / 2; step != 0; step >>= 1)
+            if (lds.coff[set][c + step] - A0 <= at) c += step;
+        A[k] = lds.src[set][c] + at - (lds.coff[set][c] - A0);
+        raw[k] = __builtin_amdgcn_raw_buffer_load_b32(rs, word_at(A[k], last), 0, 0);
+    }
+    // (Every load is waited for here: one left in flight on some lane made the
+    // rounds that gather nothing wait at this place for their last stores,
+    // 1.5% on the layer at 1024-symbol chunks and 4% on the GEMM.)
+#pragma unroll
+    for (uint32_t k = 0; k < kTileBatch; ++k) consume(raw[k]);
+    uint32_t* const top = lds.tile + kRunTileWords - 1;
+#pragma unroll
+    for (uint32_t k = 0; k < kTileBatch; ++k) {
+        const uint32_t j = k * kThreads + tid;
+        if (j >= kRunTileWords) continue;
+        const uint32_t v = raw[k] >> (8 * ((A[k] - word_at(A[k], last)) & 3u));
+        *(top - j) = A[k] < T.packed_n32 ? be_word(v, T.packed_n32 - A[k], 0) : 0u;
+    }
+}
+
 // Chunks [ca, cb) of tensor T (all of them below n_jobs).
 template <int kMode, int kGroup, class Args>
 __device__ void spec_piece(SpecLds& lds, const Tables& tb, bool global_esc, const Args& args,
@@ -3573,7 +3644,7 @@ __device__ void spec_piece(SpecLds& lds, const Tables& tb, bool global_esc, cons
     }
     uint32_t b = 0;
     uint32_t jj = 0;
-    SpecTab tab = spec_tab_commit(TF, T, lds, b, ca, cb, 0u, 0u, false, S, smagic, lane, w, &jj);
+    SpecTab tab = spec_tab_commit<gathers(kMode)>(TF, T, lds, b, ca, cb, 0u, 0u, false, S, smagic, lane, w, &jj);
     uint32_t c0 = ca;     // chunk of the round's first segment
     uint32_t p0 = 0;      // chunk bit where its first codeword starts (k0 > 0)
     GemmAcc gacc;         // fused GEMM without a ring: this wave's partial sums
@@ -3607,6 +3678,10 @@ __device__ void spec_piece(SpecLds& lds, const Tables& tb, bool global_esc, cons
         const uint32_t k0n = tab.k0n;
         const uint32_t offn = tab.offn;
         const uint32_t A0n = offn + k0n * (S / 8);
+        if (gathers(kMode) && tab.apart != 0u) {
+            spec_tile_gather(T, lds, b, A0, tid);
+            __syncthreads();  // the round's words are in the tile
+        }
         __builtin_amdgcn_s_setprio(3);
         if (more) {
             spec_tile_issue(raw, T, A0n, tid);
@@ -3748,7 +3823,7 @@ __device__ void spec_piece(SpecLds& lds, const Tables& tb, bool global_esc, cons
         uint32_t jjn = 0;
         if (more) {
             spec_tile_commit(raw, T, A0n, tid, lds.tile);
-            tabn = spec_tab_commit(TF, T, lds, b ^ 1u, c0n, cb, k0n, offn, true, S, smagic, lane, w,
+            tabn = spec_tab_commit<gathers(kMode)>(TF, T, lds, b ^ 1u, c0n, cb, k0n, offn, true, S, smagic, lane, w,
                                    &jjn);
         }
         if constexpr (kMode == kModeGemmTile) consume(sm_touch);
@@ -3841,9 +3916,9 @@ __device__ void spec_piece(SpecLds& lds, const Tables& tb, bool global_esc, cons
     if (fall_from < 0) {
         if (tid < lead) store_one<kMode>(T, args.gemv, a0 + tid, stage[tid]);
     } else {
-        // A chunk that does not hold its symbols, or chunks not back to back:
-        // from fall_from on, each chunk is decoded by one thread codeword by
-        // codeword (exact on any input).
+        // A chunk that does not hold its symbols (GEMM modes: or chunks not
+        // back to back): from fall_from on, each chunk is decoded by one
+        // thread codeword by codeword (exact on any input).
         run_fallback<kMode>(tb, args, T, fall_from / cs, cb, fall_from);
     }
     if constexpr (keeps_tile_sums(kMode)) gemm_finish(gacc, args.gemv, stage);

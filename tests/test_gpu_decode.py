@@ -209,3 +209,24 @@ def test_chunks_below_1024_symbols(chunk, n, monkeypatch):
     assert torch.equal(u8, ((want.int() >> 7) & 0xFF).to(torch.uint8))
     monkeypatch.setenv("AIMG_SPEC_RUNS", "0")
     assert torch.equal(decode_bf16([t])[0].cpu().view(torch.int16), want)
+
+
+@pytest.mark.parametrize("kind", ["gap", "padded", "shuffled"])
+@pytest.mark.parametrize("chunk", [128, 512, 1000, 1024, 8192])
+def test_chunks_not_back_to_back(chunk, kind):
+    """Padded streams and streams in another chunk order: bf16, exponent bytes
+    and the fused GEMV (against 64 bits: one rounding a term at most)."""
+    from afterimage_amd import workloads
+    from afterimage_amd.runtime.compressed_store import compress_layer
+    from afterimage_amd.runtime.device import DeviceTensor, decode_bf16, decode_gemv, decode_u8
+    from tests.edited_streams import edited
+    W = workloads.bf16_normal((2003, 1000), chunk, 0.02, outlier_frac=1e-3)
+    layer = compress_layer(W, chunk_size=chunk)
+    t = DeviceTensor.from_encoded(edited(layer.encoded, kind), layer.sign_mantissa, "cuda")
+    want = W.reshape(-1).view(torch.int16)
+    assert torch.equal(decode_bf16([t])[0].cpu().reshape(-1).view(torch.int16), want)
+    assert torch.equal(decode_u8([t])[0].cpu().reshape(-1), ((want.int() >> 7) & 0xFF).to(torch.uint8))
+    x = torch.randn(3, 1000, generator=torch.Generator().manual_seed(chunk)).to(torch.bfloat16)
+    y = decode_gemv(t, x.cuda(), 2003, 1000).cpu().double()
+    bound = 1000 * 2.0 ** -24 * (x.double().abs() @ W.double().abs().t())
+    assert bool(((y - x.double() @ W.double().t()).abs() <= bound).all())

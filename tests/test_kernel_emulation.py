@@ -609,12 +609,11 @@ def test_fused_gemm_ring(emu, rows, cols, chunk, n_x, cus):
           cus=cus, mode="gemm-ring")
 
 
-# The same GEMMs of streams that leave the ring early for the exact path: a
-# workgroup's ring is then flushed with whatever rows it holds, and the exact
-# path adds the rest, each weight once. Chunks swapped, a gap before one, an
-# empty one (in the middle, and first of a workgroup's), a last one cut short,
-# and a re-packed stream whose chunks all miss their last byte (back to back,
-# so that rounds decode until one does not hold its symbols).
+# The same GEMMs of edited streams. Chunks that hold their symbols in another
+# order or apart from each other decode in rounds that gather their words; an
+# empty chunk, one cut short, or chunks that all miss their last byte make a
+# workgroup leave its ring for the exact path, the ring flushed with whatever
+# rows it holds, each weight taken once.
 
 def _gemm_edited(emu, name, rows, cols, chunk, n_x, kind, mode, cus):
     import oracle
@@ -638,7 +637,7 @@ def _gemm_edited(emu, name, rows, cols, chunk, n_x, kind, mode, cus):
 
 
 @pytest.mark.parametrize("kind", LOSSLESS + LOSSY)
-def test_fused_gemm_ring_exact_path(emu, kind):
+def test_fused_gemm_ring_edited(emu, kind):
     _gemm_edited(emu, "ringx_%s" % kind, 40, 5120, 4096, 6, kind, "gemm-ring", 1)
 
 
@@ -666,3 +665,47 @@ def test_spec_small_chunks_gemv(emu):
 @pytest.mark.parametrize("rows,cols,batch", [(900, 8, 2), (40, 504, 1), (120, 136, 4)])
 def test_gemv_short_rows(emu, rows, cols, batch):
     _gemv(emu, "gshort_%d" % cols, rows, cols, 1024, batch, 31, cus=1)
+
+
+# Rounds whose chunks are not back to back: swapped, padded and shuffled
+# streams, in chunks of a few segments (many to a table, which ends before the
+# round's segments do) and of more segments than a round (rounds that start
+# inside a chunk), one-bit codes (80-bit segments), and no slack bytes after
+# the last chunk.
+
+@pytest.mark.parametrize("chunk,n,kind", [
+    pytest.param(chunk, n, kind, marks=[] if kind in some else [full])
+    for chunk, n, some in ((128, 20003, ("shuffled",)), (1000, 30000, ("gap-late", "padded")),
+                           (8192, 40000, ("swapped", "padded")))
+    for kind in LOSSLESS])
+def test_spec_chunks_not_back_to_back(emu, chunk, n, kind):
+    W = workloads.bf16_normal((n,), chunk, 0.02, outlier_frac=1e-3)
+    layer = compress_layer(W, chunk_size=chunk)
+    enc = edited(layer.encoded, kind)
+    enc.packed = enc.packed[: int((enc.chunk_offsets + enc.chunk_nbytes).max())]
+    name = "spapart_%d_%s" % (chunk, kind)
+    _write(emu[1] / name, enc, W.view(torch.int16).numpy(), layer.sign_mantissa.numpy())
+    _run(emu, name, "bf16", cus=1)
+
+
+@pytest.mark.parametrize("kind", ["padded", "shuffled"])
+def test_spec_chunks_not_back_to_back_one_bit_codes(emu, kind):
+    exps = np.random.default_rng(3).integers(0, 2, 128 * 300 + 40)
+    enc = edited(encode_chunked(torch.as_tensor(exps), chunk_size=128), kind)
+    _write(emu[1] / ("spapart1_" + kind), enc, exps.astype(np.uint8))
+    _run(emu, "spapart1_" + kind, "u8", cus=1)
+
+
+@full
+@pytest.mark.parametrize("kind", LOSSY)
+def test_spec_small_chunks_malformed(emu, kind):
+    # Chunks of 512 symbols, empty and cut short: the same bytes as chunk by
+    # chunk and as the oracle.
+    rng = np.random.default_rng(34)
+    enc = encode_chunked(torch.as_tensor(rng.integers(100, 140, 512 * 16)), chunk_size=512)
+    _malformed(emu, "spsm_" + kind, edited(enc, kind))
+
+
+@pytest.mark.parametrize("kind", ["padded", "shuffled"])
+def test_spec_gemv_chunks_not_back_to_back(emu, kind):
+    _gemm_edited(emu, "gvapart_" + kind, 70, 264, 136, 3, kind, "gemv", 1)
