@@ -4450,21 +4450,39 @@ int check_tensor(const aimg_tensor& t) {
     return normal.m == 0 && tiny.m == 0 ? AIMG_OK : fail_gemm_layout();
 }
 
-// Whether the ring serves an n_x-row GEMM faster than the modes without it
-// (microseconds without, with; 1024-symbol chunks unless said). Rows of more
-// than kGemmPieceMaxCols columns: but for a handful of rows (4x20480, 16 rows
-// of x: 37, 18; 3000x20480: 249, 77; 20x9000, 5 rows: 26, 22; 8x12000 at
-// 16384 symbols: 23, 26). Shorter ones: X is read once a piece of 2048 groups
-// without the ring, which costs more with more rows of x and more columns.
-// 16 rows: 30000x1000 43, 48; 30000x1400 61, 59; 8000x2048 36, 32; 800x5120
-// 26, 23. 5 rows: 8000x2048 31, 32; 30000x2048 71, 70; 800x5120 21, 23;
-// 2000x4096 26, 25; 4096x4096 at 65536 symbols 38, 32. n_x 0: not asked.
-bool ring_pays(int64_t n_symbols, int64_t rows, int64_t cols, int n_x) {
+// Whether the ring serves an n_x-row GEMM faster than the modes without it.
+// The ring reads x once per 16 rows of W, the others once a round (or once a
+// piece of 2048 groups, rows of up to kGemmPieceMaxCols columns), which costs
+// more with more rows of x, more columns and more rounds a workgroup; against
+// it stand the packing launch and the workspace, and few rounds a workgroup to
+// take x once for. Time without the ring over time with it, 5, 9 and 16 rows of
+// x, on both sides of each line:
+//   rows of up to 8192 columns, chunks of several rounds (65536 symbols):
+//     12x2048 0.98 0.97 0.99, 40x2048 1.10 1.16 1.27, 16x4096 1.25 1.36 1.62;
+//   smaller chunks (1024 symbols; 16384 in brackets): 600x4096 0.87 0.95 1.06
+//     (0.87 0.87 0.90), 2000x4096 1.11 1.19 1.39 (0.96 1.03 1.16), 600x6144
+//     0.93 1.02 1.19, 1000x6144 1.02 1.11 1.37, 2000x6144 0.96 1.06 1.29,
+//     4000x6144 1.27 1.44 1.78, 2000x2048 0.95 0.96 0.98, 4000x2048 0.96 1.02
+//     1.12;
+//   9000 columns (any chunk but 65536 symbols: there 1.1 to 1.4): 16 rows 0.86
+//     to 1.09, 24 rows 1.10 to 1.29;
+//   longer rows, chunks of about a round, one workgroup a CU at most: 100x17408
+//     at 16384 symbols 0.98 1.01 1.19, 300x17408 1.39 1.45 1.77, 100x12288 at
+//     8192 0.96 1.00 1.11, 200x12288 1.30 1.37 1.61; at 1024 and 4096 symbols
+//     1.02 to 1.9 from 12 rows on.
+// n_x 0: not asked.
+bool ring_pays(int64_t n_symbols, int64_t rows, int64_t cols, int64_t chunk_size, int n_x) {
     if (n_x == 0) return true;
+    const bool rounds = chunk_size > (1 << 15);  // several a chunk
+    if (cols <= kGemmPieceMaxCols) {
+        if (cols < (n_x > 8 ? 2048 : 4096)) return false;
+        if (rounds) return n_symbols >= (1 << 16);
+        return n_symbols >= (n_x <= 8 ? 1 << 24 : cols < 4096 ? 1 << 23 : 1 << 22);
+    }
     if (rows < 12 && n_x <= 8) return false;
-    if (cols > kGemmPieceMaxCols) return true;
-    if (n_x > 8) return cols >= 2048;
-    return cols >= 4096 && n_symbols >= (int64_t{1} << 23);
+    if (cols <= 10240) return rows >= 24 || rounds;
+    const bool a_round = chunk_size >= 8192 && chunk_size <= (1 << 14);
+    return !(n_x <= 8 && a_round && (n_symbols + chunk_size - 1) / chunk_size <= cu_count());
 }
 
 // Rows of a workgroup's ring for a rows x cols weight in chunks of
@@ -4763,7 +4781,7 @@ extern "C" int aimg_gemm_workspace_nbytes(const aimg_tensor* t, int64_t rows, in
     if (n_x < 0 || n_x > aimg::kGemmMaxRows)
         return fail(AIMG_ERR_INVALID_ARGUMENT, "n_x must be in 0.." + std::to_string(aimg::kGemmMaxRows));
     *nbytes = 0;
-    if (cols % 8 != 0 || t->chunk_size < 8 || !aimg::ring_pays(t->n_symbols, rows, cols, n_x)) return AIMG_OK;
+    if (cols % 8 != 0 || t->chunk_size < 8 || !aimg::ring_pays(t->n_symbols, rows, cols, t->chunk_size, n_x)) return AIMG_OK;
     *nbytes = aimg::plan_ring(t->n_symbols, cols, t->chunk_size).nbytes;
     return AIMG_OK;
 }

@@ -22,6 +22,7 @@ from __future__ import annotations
 import collections
 import ctypes
 import dataclasses
+import functools
 import hashlib
 import threading
 import weakref
@@ -570,8 +571,8 @@ def _fused(t: DeviceTensor, x: torch.Tensor, rows: int, cols: int, y: torch.Tens
     d[0] = _descriptor(t, None, t.n_symbols)
     with torch.cuda.device(dev):
         ws = None
-        if entry == "aimg_decode_gemm_bf16" and cols >= 2048:  # (shorter rows take none)
-            ws = _gemm_workspace(d, rows, cols, b, dev)
+        if entry == "aimg_decode_gemm_bf16":
+            ws = _gemm_workspace(t, rows, cols, b, dev)
         if ws is not None:
             zero_y = y is None
             if zero_y:
@@ -587,17 +588,25 @@ def _fused(t: DeviceTensor, x: torch.Tensor, rows: int, cols: int, y: torch.Tens
     return y
 
 
-def _gemm_workspace(d, rows: int, cols: int, b: int, dev) -> torch.Tensor | None:
+@functools.lru_cache(maxsize=1024)
+def _gemm_workspace_nbytes(n_symbols: int, chunk_size: int, rows: int, cols: int, b: int) -> int:
+    d = _native.AimgTensor(n_symbols=n_symbols, chunk_size=chunk_size)
+    nbytes = ctypes.c_size_t(0)
+    _native.check(_native.lib().aimg_gemm_workspace_nbytes(ctypes.byref(d), rows, cols, b, ctypes.byref(nbytes)))
+    return nbytes.value
+
+
+def _gemm_workspace(t: DeviceTensor, rows: int, cols: int, b: int, dev) -> torch.Tensor | None:
     """Scratch memory of one fused GEMM, from torch's caching allocator on the
     current stream (which the launch uses, so the block goes back to the
     allocator in stream order); None where the shape takes none or the memory
-    is not to be had (the GEMM then runs without it, slower)."""
-    nbytes = ctypes.c_size_t(0)
-    _native.check(_native.lib().aimg_gemm_workspace_nbytes(d, rows, cols, b, ctypes.byref(nbytes)))
-    if nbytes.value == 0:
+    is not to be had (the GEMM then runs without it, slower). Its size depends
+    on the sizes alone (asked for once each: 1.5 us of a call)."""
+    nbytes = _gemm_workspace_nbytes(t.n_symbols, t.chunk_size, rows, cols, b)
+    if nbytes == 0:
         return None
     try:
-        return torch.empty(nbytes.value, dtype=torch.uint8, device=dev)
+        return torch.empty(nbytes, dtype=torch.uint8, device=dev)
     except torch.OutOfMemoryError:
         return None
 

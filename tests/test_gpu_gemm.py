@@ -5,6 +5,8 @@ step_k + 1 positions at :2554-2556). The weights decode bit-exact, so the
 reference product is the fp32 matmul of the original bf16 weights; the
 result must agree within rel 1e-2 / abs 1e-3 (bf16 products, fp32 sums in
 no fixed order, then bf16 for the API's result)."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -12,7 +14,7 @@ import torch
 from afterimage_amd import _native, workloads
 from afterimage_amd.runtime.compressed_store import (compress_layer, decompress_linear_gpu,
                                                      decompress_matvec_gpu)
-from afterimage_amd.runtime.device import GEMM_MAX_ROWS, DeviceTensor, decode_gemm
+from afterimage_amd.runtime.device import GEMM_MAX_ROWS, DeviceTensor, _descriptor, decode_gemm
 from tests.edited_streams import LOSSLESS, edited
 
 pytestmark = pytest.mark.gpu
@@ -136,6 +138,22 @@ def _ring_bound(W, x):
     return W.shape[1] * 2.0 ** -24 * (x.double().abs() @ W.double().abs().t()) + 1e-30
 
 
+def _ring(t, x, rows, cols):
+    """The GEMM through a ring whatever the shape, into a y of NaN."""
+    d = (_native.AimgTensor * 1)()
+    d[0] = _descriptor(t, None, t.n_symbols)
+    n = ctypes.c_size_t(0)
+    lib = _native.lib()
+    _native.check(lib.aimg_gemm_workspace_nbytes(d, rows, cols, 0, ctypes.byref(n)))
+    assert n.value > 0
+    ws = torch.empty(n.value, dtype=torch.uint8, device="cuda")
+    y = torch.full((x.shape[0], rows), float("nan"), device="cuda")
+    _native.check(lib.aimg_decode_gemm_bf16_ws(d, rows, cols, x.data_ptr(), x.shape[0], y.data_ptr(), 1,
+                                               ws.data_ptr(), ws.numel(),
+                                               torch.cuda.current_stream().cuda_stream))
+    return y
+
+
 @pytest.mark.parametrize("shape,chunk,n_x", [((31, 18000), 5000, 12), ((4, 20480), 1024, 16),
                                              ((1, 8200), 65536, 1), ((700, 2056), 1024, 9),
                                              ((2100, 4104), 8192, 5), ((5120, 2048), 1000 + 24, 16),
@@ -148,8 +166,8 @@ def test_ring(shape, chunk, n_x):
     layer = compress_layer(W, chunk_size=chunk)
     x = _x(n_x, shape[1], 5)
     t = DeviceTensor.from_encoded(layer.encoded, layer.sign_mantissa, "cuda")
-    for _ in range(2):  # the second call finds the first one's workspace
-        y = decode_gemm(t, x.cuda(), *shape).cpu().double()
+    for call in (_ring, decode_gemm, _ring):  # the last finds a used workspace
+        y = call(t, x.cuda(), *shape).cpu().double()
         assert bool(((y - x.double() @ W.double().t()).abs() <= _ring_bound(W, x)).all())
 
 
@@ -164,9 +182,10 @@ def test_ring_infinite_x():
     x = _x(6, 10000, 2)
     x[2, col] = float("inf")
     t = DeviceTensor.from_encoded(layer.encoded, layer.sign_mantissa, "cuda")
-    y = decode_gemm(t, x.cuda(), 64, 10000).cpu()
-    assert bool(torch.isposinf(y[2]).all())
-    assert bool(torch.isfinite(y[[0, 1, 3, 4, 5]]).all())
+    for call in (_ring, decode_gemm):
+        y = call(t, x.cuda(), 64, 10000).cpu()
+        assert bool(torch.isposinf(y[2]).all())
+        assert bool(torch.isfinite(y[[0, 1, 3, 4, 5]]).all())
 
 
 @pytest.mark.parametrize("kind", LOSSLESS)
@@ -178,5 +197,5 @@ def test_ring_chunks_not_back_to_back(shape, chunk, n_x, kind):
     layer = compress_layer(W, chunk_size=chunk)
     x = _x(n_x, shape[1], 6)
     t = DeviceTensor.from_encoded(edited(layer.encoded, kind), layer.sign_mantissa, "cuda")
-    y = decode_gemm(t, x.cuda(), *shape).cpu().double()
+    y = _ring(t, x.cuda(), *shape).cpu().double()
     assert bool(((y - x.double() @ W.double().t()).abs() <= _ring_bound(W, x)).all())

@@ -304,3 +304,20 @@ def test_build_index_validates_before_launching():
     arr[0].index = 4096  # the shared checks: null device pointers
     assert lib.aimg_build_index(arr, 1, None) == _native.AIMG_ERR_INVALID_ARGUMENT
     assert b"null" in lib.aimg_last_error()
+
+
+@pytest.mark.parametrize("rows,cols,chunk,n_x,ring", [
+    (5120, 17408, 65536, 16, True), (151936, 5120, 1024, 8, True), (4096, 4096, 65536, 5, True),
+    (4, 20480, 1024, 16, True), (24, 9000, 16384, 5, True), (300, 17408, 16384, 5, True),
+    # Few rounds a workgroup, where packing x and the workspace cost more.
+    (64, 2048, 1024, 9, False), (64, 4096, 1024, 9, False), (600, 4096, 16384, 16, False),
+    (16, 9000, 16384, 8, False), (4, 9000, 1024, 16, False), (100, 17408, 16384, 5, False),
+    (100, 12288, 8192, 5, False), (2000, 6144, 16384, 5, False), (8, 17408, 65536, 8, False),
+])
+def test_gemm_takes_a_workspace_where_it_pays(rows, cols, chunk, n_x, ring):
+    d = (_native.AimgTensor * 1)()
+    d[0].n_symbols = rows * cols
+    d[0].chunk_size = chunk
+    n = ctypes.c_size_t(1)
+    _native.check(_native.lib().aimg_gemm_workspace_nbytes(d, rows, cols, n_x, ctypes.byref(n)))
+    assert (n.value > 0) == ring
