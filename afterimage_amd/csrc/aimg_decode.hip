@@ -4303,15 +4303,24 @@ int launch_run(Batch& B, hipStream_t s) {
 }
 
 // Workgroups of a speculative launch: one per chunk up to two per CU, and one
-// per CU where that leaves none more than about a round of segments: it then
+// per CU where that leaves none more than one round of segments: it then
 // decodes as long alone as with another beside it, and half of the start-ups
 // and table loads fall away (1024x3072 at 4096-symbol chunks 12.1 -> 11.6 us,
 // 400x1000 at 1024 12.8 -> 11.0; one workgroup per round, 96 of them, 18.4).
-int64_t spec_grid(const Batch& B, int64_t chunks, int64_t slots, bool gemm) {
+// With a second round for some it is slower than two workgroups beside each
+// other: 8000x1000 bf16 at 512, 2048 and 5000 symbols 19.2, 19.0 and 19.9 us
+// against 15.6, 15.6 and 16.1. Segments are counted as a chunk's bits over their
+// length and a half for its last one, with the length of one-bit codes where
+// the codes average fewer than two bits (the table is in device memory).
+int64_t spec_grid(const Batch& B, int64_t chunks, int64_t elements, int64_t slots, bool gemm) {
     int64_t bits = 0;
     for (int d = 0; d < B.m; ++d) bits += 8 * B.args.t[d].packed_nbytes;
-    const bool one_round = bits / (static_cast<int64_t>(kThreads) * kMaxSegBits) + 1 < slots / 2;
-    int64_t most = one_round && slots > 1 ? slots / 2 : slots;
+    const int64_t S = bits < 2 * elements ? segment_bits(1) : kMaxSegBits;
+    const int64_t half = slots > 1 ? slots / 2 : slots;
+    const int64_t per = (chunks + half - 1) / half;
+    const bool one_round = per <= static_cast<int64_t>(kSpecChunks) &&
+                           per * (bits / chunks) / S + per / 2 <= kThreads - 4;
+    int64_t most = one_round ? half : slots;
     // A wave's worth of segments at least (a tiny tensor's chunks of a few
     // segments each would load the decode table once a chunk). The fused
     // GEMM's rings are sized for a workgroup a chunk.
@@ -4336,7 +4345,7 @@ int launch_spec(Batch& B, hipStream_t s) {
     }
     B.args.total_items = elements;
     const int64_t slots = static_cast<int64_t>(cu_count()) * kBlocksPerCu;
-    const int64_t grid = spec_grid(B, chunks, slots, is_gemm(kMode));
+    const int64_t grid = spec_grid(B, chunks, elements, slots, is_gemm(kMode));
     // A full grid: workgroups b and b + grid / 2 share a CU and split its share.
     B.args.strided = grid == slots ? 1 : 0;
     constexpr int kVecGroup = kMode == kModeU8 ? 16 : 8;

@@ -306,6 +306,10 @@ template <typename K, typename... A>
 inline void emu_launch(K kernel, dim3 g, dim3 b, A... args) {
     gridDim = {g.x, 1, 1};
     blockDim = {b.x, 1, 1};
+    if (getenv("AIMG_EMU_GRID")) {  // print the launch's workgroups instead
+        printf("grid %u: ok\n", g.x);
+        exit(0);
+    }
     for (unsigned blk = 0; blk < g.x; ++blk) {
         emu::Block B(b.x);
         emu::g_block = &B;

@@ -81,13 +81,14 @@ def _write(d, enc, expect, sm=None):
         f.write("%d %d %d %d\n" % (enc.max_bits, enc.chunk_size, enc.n_symbols, len(enc.chunk_offsets)))
 
 
-def _run(emu, name, mode, index="", runs=None, strided=None, cus=None, copies=None, spec=None):
+def _run(emu, name, mode, index="", runs=None, strided=None, cus=None, copies=None, spec=None, grid=None):
     exe, d = emu
     env = dict(os.environ, ASAN_OPTIONS="detect_leaks=0:abort_on_error=0")
     env.pop("AIMG_SEGMENT_RUNS", None)
     env.pop("AIMG_RUN_STRIDED", None)
     env.pop("AIMG_EMU_CUS", None)
     env.pop("AIMG_EMU_COPIES", None)
+    env.pop("AIMG_EMU_GRID", None)
     env.pop("AIMG_SPEC_RUNS", None)
     env.pop("AIMG_CHUNK_SPLIT", None)
     if spec is not None:
@@ -102,9 +103,12 @@ def _run(emu, name, mode, index="", runs=None, strided=None, cus=None, copies=No
         env["AIMG_SEGMENT_RUNS"] = runs
     if strided is not None:
         env["AIMG_RUN_STRIDED"] = strided
+    if grid is not None:
+        env["AIMG_EMU_GRID"] = "1"  # the first launch's workgroups, not run
     args = [exe, str(d / name), mode] + ([index] if index else [])
     r = subprocess.run(args, capture_output=True, text=True, env=env, timeout=1800)
     assert r.returncode == 0 and ": ok" in r.stdout, (r.stdout + r.stderr)[-4000:]
+    assert grid is None or r.stdout.startswith("grid %d:" % grid), r.stdout
 
 
 def _u8(emu, name, exps, chunk_size, index="", cus=None, spec=None):
@@ -709,3 +713,21 @@ def test_spec_small_chunks_malformed(emu, kind):
 @pytest.mark.parametrize("kind", ["padded", "shuffled"])
 def test_spec_gemv_chunks_not_back_to_back(emu, kind):
     _gemm_edited(emu, "gvapart_" + kind, 70, 264, 136, 3, kind, "gemv", 1)
+
+
+@pytest.mark.parametrize("chunk,chunks,one_bit,grid", [
+    (512, 2 * 48, False, 2), (512, 2 * 62, False, 4), (1024, 2 * 28, False, 2), (1024, 2 * 33, False, 4),
+    (128, 2 * 64, False, 2), (128, 2 * 66, False, 4), (1024, 2 * 36, True, 2), (1024, 2 * 42, True, 4),
+])
+def test_spec_grid(emu, chunk, chunks, one_bit, grid):
+    # One workgroup on each of two CUs where each has at most one round of
+    # segments (168 bits, 80 of one-bit codes), else two.
+    n = chunk * chunks
+    if one_bit:
+        exps = np.random.default_rng(5).integers(0, 2, n)
+    else:
+        W = workloads.bf16_normal((n,), 6, 0.02)
+        exps = (W.view(torch.int16).numpy().astype(np.int32) >> 7) & 0xFF
+    enc = encode_chunked(torch.as_tensor(exps), chunk_size=chunk)
+    _write(emu[1] / "grid", enc, exps.astype(np.uint8))
+    _run(emu, "grid", "u8", cus=2, grid=grid)
