@@ -143,8 +143,8 @@ enum Mode : int {
     kModeIndex = 4, // the segment index: each segment's first boundary and codewords
     kModeGemm = 5,      // Y += X W^T for up to 16 rows of X, W decoded on the fly (MFMA)
     kModeGemmRows = 6,  // kModeGemm for rows of more than kGemmPieceMaxCols columns
-    kModeGemvShort = 8, // kModeGemv (batch 1 too) for rows of fewer than kGemvShortCols columns
     kModeGemmTile = 7,  // kModeGemm through a ring of exponents in a workspace, 16 whole rows at a time
+    kModeGemvShort = 8, // kModeGemv (batch 1 too) for rows of fewer than kGemvShortCols columns
 };
 constexpr bool is_gemv(int mode) {
     return mode == kModeGemv || mode == kModeGemv1 || mode == kModeGemvShort;
@@ -168,7 +168,10 @@ constexpr uint32_t kNoIndex = 0xFFFFFFFFu;
 constexpr int kGemvMaxBatch = 4;
 // Rows of fewer columns (a wave's 512 elements at one store step) take a mode
 // of their own: their code in the other two made registers spill (5120x17408
-// with 4 rows of x 87.3 -> 91.3 us).
+// with 4 rows of x 87.3 -> 91.3 us). One row of x runs through its code for
+// four: code of its own for it took 36 us instead of 38 for 30 M weights at
+// 1024-symbol chunks, but its registers spill in the chunk kernel, 1% at 2 and
+// 4 rows of x and 65536 symbols.
 constexpr int64_t kGemvShortCols = 512;
 // Rows of x (tokens) of the fused decode -> GEMM: one MFMA tile's 16.
 constexpr int kGemmMaxRows = 16;
@@ -944,7 +947,6 @@ __device__ __forceinline__ uint32_t wave_scan_incl_f32(uint32_t v) {
     return __float_as_uint(x);
 }
 
-// v of the lane below (0 in lane 0; every lane active).
 // Inclusive fp32 scan over the wave that starts anew at each row: pos lanes
 // below this one belong to its row (every lane active).
 __device__ __forceinline__ float wave_rows_scan_f32(float v, uint32_t pos, uint32_t lane) {
@@ -961,6 +963,7 @@ __device__ __forceinline__ float wave_rows_scan_f32(float v, uint32_t pos, uint3
     return v;
 }
 
+// v of the lane below (0 in lane 0; every lane active).
 __device__ __forceinline__ uint32_t lane_below(uint32_t v) { return dpp<0x138>(v); }
 
 __device__ __forceinline__ uint32_t block_scan_excl(uint32_t v, uint32_t* s_wsum) {
@@ -1235,10 +1238,13 @@ __device__ __forceinline__ void gemv_round_whole(const uint2 (&sm)[kStoreBatch],
             acc_row = er + 1;
         } else {
             // Rows shorter than a wave's 512 elements: a row's lanes are
-            // summed in the wave, and its last lane adds the sum (one atomic a
-            // lane instead took 271 us for 30000x256 with 4 rows of x, and
-            // 1429 for 10000x300 at 8192-symbol chunks: lanes of a row, and
-            // waves of a round, wait for each other at one address).
+            // summed in the wave, and its last lane adds the sum (with one
+            // atomic a lane, lanes of a row and waves of a round wait for each
+            // other at one address). 30 M weights at 1024-symbol chunks, 1 and
+            // 4 rows of x, one atomic a lane against this: 504 columns 422 and
+            // 1353 us, 38 and 48; 40 columns 184 and 643, 39 and 49; 16 columns
+            // 100 and 330, 39 and 56; 8 columns, a lane a row, 38 and 75, 41
+            // and 75.
             const uint32_t pos = lc / kGroup < lane ? lc / kGroup : lane;
             const bool end = lane == 63 || lc + kGroup >= cols;
 #pragma unroll
@@ -4322,8 +4328,10 @@ int64_t spec_grid(const Batch& B, int64_t chunks, int64_t elements, int64_t slot
                            per * (bits / chunks) / S + per / 2 <= kThreads - 4;
     int64_t most = one_round ? half : slots;
     // A wave's worth of segments at least (a tiny tensor's chunks of a few
-    // segments each would load the decode table once a chunk). The fused
-    // GEMM's rings are sized for a workgroup a chunk.
+    // segments each would load the decode table once a chunk: kernel time of
+    // 2000, 5000, 20000 and 100000 symbols in chunks of 128, a workgroup a
+    // chunk 10.3, 10.4, 10.6 and 10.9 us, so 9.2, 9.8, 10.6 and 11.0). The
+    // fused GEMM's rings are sized for a workgroup a chunk.
     if (!gemm) {
         const int64_t waves = bits / (int64_t{64} * kMaxSegBits) + 1;
         most = waves < most ? waves : most;
@@ -4373,7 +4381,9 @@ constexpr uint32_t kSpecMaxTpc = 128;
 // 17408x5120 at 512 symbols bf16 120 -> 71 us, GEMV of 1 and 4 rows of x 153
 // -> 79 and 213 -> 100, of 4 rows at 1000 symbols 173 -> 96; 3001x4099
 // exponent bytes at 512, 256 and 128 symbols 20.5 -> 16.8, 32.4 -> 22.1 and
-// 57 -> 33.
+// 57 -> 33; 17408x5120 at 128 symbols bf16 409 -> 184, GEMV of 1 and 4 rows of
+// x 465 -> 204 and 589 -> 224. (One layout is slower by more than 3%: bf16 at
+// 1000 symbols in a random chunk order, 90 -> 99.)
 constexpr int32_t kSpecMinChunk = 128;
 
 template <int kMode>
