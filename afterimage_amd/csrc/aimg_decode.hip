@@ -1588,8 +1588,9 @@ __device__ __forceinline__ void gemm_round_rows(const DevTensor& T, const GemvAr
 // with 8 rows 964 -> 684 us. What bounds it now: without the products the
 // layer takes 65 us and the head 472; the exponents are written once and read
 // once more past the L2 (82 KB a workgroup at 5120 columns, 64 workgroups an
-// L2 of 4 MB), so the memory traffic is the bf16 decode's, and a workgroup
-// that waits for it leaves its CU to one decoding workgroup. Tiles of 8 or 4
+// L2 of 4 MB; 434 MB past it for the layer, 309 for its bf16 decode), and a
+// workgroup that waits for it (half of the wave cycles) leaves its CU to one
+// decoding workgroup. Tiles of 8 or 4
 // rows, which the L2 would hold, cost more in passes (115 and 128 us); so did
 // a first tile cut short in half of the workgroups, to put their passes at
 // different times (109).

@@ -154,9 +154,11 @@ int aimg_decode_gemm_bf16(const aimg_tensor* t, int64_t rows, int64_t cols, cons
  * pass through `workspace`, so that x is read once per 16 rows of W; up to 3
  * times faster. zero_y: y is set, not added to. aimg_gemm_workspace_nbytes
  * gives the bytes it takes on the current device for n_x rows of x (of *t,
- * n_symbols and chunk_size are read; at most 512 MiB and 16 packed rows of x),
- * or 0 where the call without a workspace is as fast or no workspace serves
- * the shape (n_x 0: the bytes for up to 16 rows, whichever is faster). A null, misaligned (16 bytes) or smaller workspace fails with
+ * n_symbols and chunk_size are read; 170 MB for a large matrix of 17408
+ * columns, 66 MB of 5120, at most 512 MiB and 16 packed rows of x), or 0 where
+ * the call without a workspace is as fast or no workspace serves the shape
+ * (n_x 0: the bytes for up to 16 rows, whichever is faster). A null,
+ * misaligned (16 bytes) or smaller workspace fails with
  * AIMG_ERR_INVALID_ARGUMENT. Its contents need no initialisation and mean
  * nothing afterwards; launches that may overlap need a workspace each.
  */
